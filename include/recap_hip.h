@@ -133,7 +133,7 @@ int recap_partial_reduce(const float* partial, int64_t banks, int64_t groups, in
 
 /* Eigenvalues (ascending, [batch, n]) and orthonormal eigenvectors (columns, [batch, n, n])
  * of the symmetrised 0.5 (a + a^T) of `batch` row-major fp32 n x n matrices, n <= 128:
- * the contract of torch.linalg.eigh.  One-sided parallel Jacobi in one workgroup per matrix;
+ * the contract of torch.linalg.eigh.  Two-sided parallel Jacobi in one workgroup per matrix;
  * eigenvectors are unique up to sign (and to a rotation within a repeated eigenvalue).
  * Replaces the torch.linalg.eigh call of closure_basis, recap/sparse/closure.py:75-81. */
 int recap_symmetric_eigen(const float* a, int64_t batch, int64_t n, float* eigenvalues,

@@ -337,7 +337,7 @@ int recap_symmetric_eigen(const float* a, int64_t batch, int64_t n, float* eigen
   REQUIRE(batch >= 1 && batch <= 65535, "bad batch %lld", (long long)batch);
   REQUIRE(n >= 1 && n <= 128, "matrix order %lld outside [1, 128]", (long long)n);
   EigenArgs e{};
-  e.a = a; e.batch = (int)batch; e.n = (int)n;
+  e.a = a; e.batch = (int)batch; e.n = (int)n; e.m = (int)(n + (n & 1));
   e.max_sweeps = 40; e.values = eigenvalues; e.vectors = eigenvectors;
   return hip_status(run_symmetric_eigen(e, as_stream(stream)), "symmetric_eigen launch");
 }

@@ -72,7 +72,7 @@ hipError_t run_basis_tables(const BasisArgs& a, int dtype, hipStream_t s);
 
 // Symmetric eigen-decomposition of the closure scatter (eigen.hip).
 struct EigenArgs {
-  const float* a; int batch, n, max_sweeps;
+  const float* a; int batch, n, m, max_sweeps;   // m = n rounded up to even
   float* values; float* vectors;                 // [batch][n], [batch][n][n] (columns)
 };
 hipError_t run_symmetric_eigen(const EigenArgs& a, hipStream_t s);
