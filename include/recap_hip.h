@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define RECAP_ABI_VERSION 8
+#define RECAP_ABI_VERSION 9
 
 enum { RECAP_OK = 0, RECAP_EINVAL = 1, RECAP_EUNSUPPORTED = 2, RECAP_EHIP = 3 };
 enum { RECAP_F16 = 1, RECAP_BF16 = 2 };
@@ -248,6 +248,38 @@ int recap_sparse_merge_attn(const void* q, int dtype, int64_t batch, int64_t hea
  * identical either way.  Calls that may overlap need separate queues.  No counterpart in
  * the reference (the external kernel schedules itself). */
 int64_t recap_attn_queue_words(void);
+
+/* The head and merge launches with a workspace: recap_block_sparse_attn and
+ * recap_sparse_merge_attn with claim queues as above (`balance` non-zero) and each long row
+ * (the text rows and a ragged last video block, from query block ds on) cut into `split`
+ * segments of its kept blocks, which separate workgroups walk and the last of them combines
+ * in segment order.  Rows below the long ones are bit-identical to those of the launches
+ * without a workspace; a long row's equal them for split 1 and otherwise differ by the
+ * rounding of another summation order, the same on every run.  recap_attn_split gives the
+ * split for a layer of `banks` heads whose other rows keep about `density` of their blocks
+ * (1: none); recap_attn_workspace_size the bytes (16-byte aligned device memory, contents
+ * ignored; the counters are zeroed on `stream`).  Calls that may overlap need separate
+ * workspaces.  No counterpart in the reference. */
+int64_t recap_attn_split(int64_t banks, int64_t n_tokens, int64_t n_video, double density);
+int64_t recap_attn_workspace_size(int64_t banks, int64_t dim, int64_t n_tokens, int64_t n_video,
+                                  int64_t split);
+int recap_block_sparse_attn_ws(const void* q, int dtype, int64_t batch, int64_t heads,
+                               int64_t dim, int64_t stride_b, int64_t stride_h,
+                               int64_t stride_n, const void* k_tiles, const void* vt_tiles,
+                               const int32_t* rowmap, const uint8_t* kernel_mask,
+                               int64_t n_tokens, int64_t n_video, float scale, void* head_out,
+                               float* head_lse, int64_t split, int balance, void* workspace,
+                               int64_t workspace_bytes, void* stream);
+int recap_sparse_merge_attn_ws(const void* q, int dtype, int64_t batch, int64_t heads,
+                               int64_t dim, int64_t stride_b, int64_t stride_h,
+                               int64_t stride_n, const void* k_tiles, const void* vt_tiles,
+                               const int32_t* rowmap, const uint8_t* kernel_mask,
+                               int64_t n_tokens, int64_t n_video, float scale, const void* go,
+                               const float* gl, const void* det, const float* dl,
+                               const float* glref, const float* center, float alpha_override,
+                               void* out, int64_t out_stride_b, int64_t out_stride_h,
+                               int64_t out_stride_n, int64_t split, int balance,
+                               void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Stage 4 ------------------------------------------------------------------------------ */
 

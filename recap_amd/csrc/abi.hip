@@ -435,9 +435,59 @@ static int attn_common(const void* q, int dtype, int64_t batch, int64_t heads, i
   a.n_tokens = (int)n_tokens; a.tb = (int)g.tb;
   // Long rows, started first: the text rows (from ds) and a ragged last video block, which
   // the selection keeps dense (recap/sparse/attention.py:88-94).
-  a.ds = (int)((n_video % kBlock) != 0 ? g.nb - 1 : g.ds);
+  a.ds = (int)(n_video % kBlock != 0 ? g.nb - 1 : g.ds);
   a.rows = (int)g.rows;
   return RECAP_OK;
+}
+
+// Workspace of a split, load-balanced attention launch: the claim queues and the long rows'
+// arrival counters (zeroed together by one fill kernel on the stream, so a captured graph
+// records no memset), then the segments' states.
+struct AttnSpace {
+  int64_t counters, bytes;  // 32-bit words to zero, and the whole size
+};
+
+static AttnSpace attn_space(int64_t banks, int64_t dim, int64_t long_rows, int64_t split) {
+  AttnSpace w;
+  const int64_t tickets = split > 1 ? banks * long_rows : 0;
+  w.counters = kQueueWords + (tickets + 63) / 64 * 64;
+  w.bytes = w.counters * 4 + tickets * split * attn_part_words((int)dim) * 8;
+  return w;
+}
+
+// First long query row (see AttnArgs::ds): the text rows and a ragged last video block.
+static int64_t first_long(const Geom& g, int64_t n_video) {
+  return n_video % kBlock != 0 ? g.nb - 1 : g.ds;
+}
+
+static int set_workspace(AttnArgs& a, int64_t dim, int64_t split, int balance, void* workspace,
+                         int64_t bytes, hipStream_t s) {
+  REQUIRE(split >= 1 && split <= kMaxSplit, "split %lld outside 1..%d", (long long)split, kMaxSplit);
+  REQUIRE(workspace != nullptr && aligned16(workspace), "workspace must be non-NULL and 16-byte aligned");
+  const AttnSpace w = attn_space(a.banks, dim, a.tb - a.ds, split);
+  REQUIRE(bytes >= w.bytes, "workspace of %lld bytes, need %lld", (long long)bytes, (long long)w.bytes);
+  unsigned* words = static_cast<unsigned*>(workspace);
+  CHECK(hip_status(run_zero_words(words, (int)w.counters, s), "attention counters reset"));
+  a.queue = balance ? words : nullptr;
+  a.split = a.tb > a.ds ? (int)split : 1;
+  a.tickets = words + kQueueWords;
+  a.part = reinterpret_cast<unsigned long long*>(words + w.counters);
+  return RECAP_OK;
+}
+
+int64_t recap_attn_split(int64_t banks, int64_t n_tokens, int64_t n_video, double density) {
+  if (banks < 1 || n_video < 1 || n_tokens < n_video || !(density > 0.0 && density <= 1.0)) return -1;
+  const Geom g = geometry(n_tokens, n_video);
+  return attn_split(banks, g.tb, first_long(g, n_video), density);
+}
+
+int64_t recap_attn_workspace_size(int64_t banks, int64_t dim, int64_t n_tokens, int64_t n_video,
+                                  int64_t split) {
+  if (banks < 1 || (dim != 64 && dim != 128) || n_video < 1 || n_tokens < n_video || split < 1 ||
+      split > kMaxSplit)
+    return -1;
+  const Geom g = geometry(n_tokens, n_video);
+  return attn_space(banks, dim, g.tb - first_long(g, n_video), split).bytes;
 }
 
 int recap_block_sparse_attn(const void* q, int dtype, int64_t batch, int64_t heads,
@@ -454,6 +504,25 @@ int recap_block_sparse_attn(const void* q, int dtype, int64_t batch, int64_t hea
   a.kmask = kernel_mask; a.ds = a.tb;
   CHECK(set_scale(a, scale));
   a.head_out = static_cast<uint16_t*>(head_out); a.head_lse = head_lse;
+  return hip_status(run_attention(a, dtype, (int)dim, kModeHead, as_stream(stream)), "attention launch");
+}
+
+int recap_block_sparse_attn_ws(const void* q, int dtype, int64_t batch, int64_t heads,
+                               int64_t dim, int64_t stride_b, int64_t stride_h,
+                               int64_t stride_n, const void* k_tiles, const void* vt_tiles,
+                               const int32_t* rowmap, const uint8_t* kernel_mask,
+                               int64_t n_tokens, int64_t n_video, float scale, void* head_out,
+                               float* head_lse, int64_t split, int balance, void* workspace,
+                               int64_t workspace_bytes, void* stream) {
+  AttnArgs a{};
+  CHECK(attn_common(q, dtype, batch, heads, dim, stride_b, stride_h, stride_n, k_tiles, vt_tiles,
+                    rowmap, n_tokens, n_video, a));
+  REQUIRE(kernel_mask && head_out && head_lse, "NULL mask or output");
+  REQUIRE(aligned16(head_out), "head_out must be 16-byte aligned");
+  a.kmask = kernel_mask;
+  CHECK(set_scale(a, scale));
+  a.head_out = static_cast<uint16_t*>(head_out); a.head_lse = head_lse;
+  CHECK(set_workspace(a, dim, split, balance, workspace, workspace_bytes, as_stream(stream)));
   return hip_status(run_attention(a, dtype, (int)dim, kModeHead, as_stream(stream)), "attention launch");
 }
 
@@ -497,16 +566,15 @@ int recap_dense_head_attn(const void* q, int dtype, int64_t batch, int64_t heads
   return hip_status(run_attention(a, dtype, (int)dim, kModeDenseHead, as_stream(stream)), "attention launch");
 }
 
-int recap_sparse_merge_attn(const void* q, int dtype, int64_t batch, int64_t heads,
-                            int64_t dim, int64_t stride_b, int64_t stride_h, int64_t stride_n,
-                            const void* k_tiles, const void* vt_tiles, const int32_t* rowmap,
-                            const uint8_t* kernel_mask, int64_t n_tokens, int64_t n_video,
-                            float scale, const void* go, const float* gl, const void* det,
-                            const float* dl, const float* glref, const float* center,
-                            float alpha_override, void* out, int64_t out_stride_b,
-                            int64_t out_stride_h, int64_t out_stride_n, uint32_t* work_queue,
-                            void* stream) {
-  AttnArgs a{};
+// Arguments of a merge launch, validated; the caller sets the queue.
+static int merge_args(const void* q, int dtype, int64_t batch, int64_t heads, int64_t dim,
+                      int64_t stride_b, int64_t stride_h, int64_t stride_n, const void* k_tiles,
+                      const void* vt_tiles, const int32_t* rowmap, const uint8_t* kernel_mask,
+                      int64_t n_tokens, int64_t n_video, float scale, const void* go,
+                      const float* gl, const void* det, const float* dl, const float* glref,
+                      const float* center, float alpha_override, void* out,
+                      int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_n,
+                      AttnArgs& a) {
   CHECK(attn_common(q, dtype, batch, heads, dim, stride_b, stride_h, stride_n, k_tiles, vt_tiles,
                     rowmap, n_tokens, n_video, a));
   CHECK(check_qkv("out", out, batch, heads, out_stride_b, out_stride_h, out_stride_n));
@@ -522,7 +590,41 @@ int recap_sparse_merge_attn(const void* q, int dtype, int64_t batch, int64_t hea
   a.dl = dl; a.glref = glref; a.center = center;
   a.use_override = alpha_override >= 0.0f ? 1 : 0;
   a.alpha_override = alpha_override;
+  return RECAP_OK;
+}
+
+int recap_sparse_merge_attn(const void* q, int dtype, int64_t batch, int64_t heads,
+                            int64_t dim, int64_t stride_b, int64_t stride_h, int64_t stride_n,
+                            const void* k_tiles, const void* vt_tiles, const int32_t* rowmap,
+                            const uint8_t* kernel_mask, int64_t n_tokens, int64_t n_video,
+                            float scale, const void* go, const float* gl, const void* det,
+                            const float* dl, const float* glref, const float* center,
+                            float alpha_override, void* out, int64_t out_stride_b,
+                            int64_t out_stride_h, int64_t out_stride_n, uint32_t* work_queue,
+                            void* stream) {
+  AttnArgs a{};
+  CHECK(merge_args(q, dtype, batch, heads, dim, stride_b, stride_h, stride_n, k_tiles, vt_tiles,
+                   rowmap, kernel_mask, n_tokens, n_video, scale, go, gl, det, dl, glref, center,
+                   alpha_override, out, out_stride_b, out_stride_h, out_stride_n, a));
   CHECK(set_queue(a, work_queue, as_stream(stream)));
+  return hip_status(run_attention(a, dtype, (int)dim, kModeMerge, as_stream(stream)), "attention launch");
+}
+
+int recap_sparse_merge_attn_ws(const void* q, int dtype, int64_t batch, int64_t heads,
+                               int64_t dim, int64_t stride_b, int64_t stride_h,
+                               int64_t stride_n, const void* k_tiles, const void* vt_tiles,
+                               const int32_t* rowmap, const uint8_t* kernel_mask,
+                               int64_t n_tokens, int64_t n_video, float scale, const void* go,
+                               const float* gl, const void* det, const float* dl,
+                               const float* glref, const float* center, float alpha_override,
+                               void* out, int64_t out_stride_b, int64_t out_stride_h,
+                               int64_t out_stride_n, int64_t split, int balance,
+                               void* workspace, int64_t workspace_bytes, void* stream) {
+  AttnArgs a{};
+  CHECK(merge_args(q, dtype, batch, heads, dim, stride_b, stride_h, stride_n, k_tiles, vt_tiles,
+                   rowmap, kernel_mask, n_tokens, n_video, scale, go, gl, det, dl, glref, center,
+                   alpha_override, out, out_stride_b, out_stride_h, out_stride_n, a));
+  CHECK(set_workspace(a, dim, split, balance, workspace, workspace_bytes, as_stream(stream)));
   return hip_status(run_attention(a, dtype, (int)dim, kModeMerge, as_stream(stream)), "attention launch");
 }
 

@@ -29,6 +29,8 @@
 // then ascending), and dense-head stores its head branch before the first block after the
 // kept ones can move the running max, so the head branch of head, dense-head and merge
 // modes is the same bit for bit.
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -63,6 +65,15 @@ __device__ inline void tile_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Wait for this wave's LDS accesses, then for every wave, with its global loads (the Q rows)
+// left in flight.
+__device__ inline void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xf | (0x7 << 4) | (0x3 << 14));  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // Each wave owns kGroups groups of 32 query rows, so every K/V fragment it reads from LDS
 // feeds kGroups MFMAs; a 128-row query block then takes kThreads threads.  kGroups = 2
 // halves the LDS reads and is correct, but at d = 128 it needs one wave per SIMD and the
@@ -71,28 +82,42 @@ constexpr int kGroups = 1;
 constexpr int kRowsPerWave = 32 * kGroups;
 constexpr int kThreads = 64 * (kBlock / kRowsPerWave);
 
-// Final normalisation and store of one query row per lane pair (lane l holds output columns
-// 32 dt + 8 q4 + 4 g .. +3 of the row), in the layout of the kernel's mode.
+// Final normalisation and store of one query row per lane pair, in the layout of the kernel's
+// mode.  Lane (g, l32) holds columns 32 dt + 8 q4 + 4 g .. +3 of its row; one exchange of
+// packed words within the lane pair gives it 8 consecutive ones, 32 dt + 16 j + 8 g .., so that
+// every access moves 16 bytes.  In merge mode the row's coarse output and refinement are all
+// requested before the first of them is used: with the loads between the stores (which the
+// compiler must keep in order: the output might be one of the inputs) each 8-byte load waited
+// out the memory's latency, 16-18 us a work item of 100-200 us; now 4.
 template <class T, int D, int MODE>
 __device__ inline void store_rows(const AttnArgs& a, int bank, int b, int h, int r, int nat,
                                   int g, const f32x16 (&oacc)[D / 32], float m, float lt) {
-  constexpr int NDT = D / 32;
+  constexpr int NV = D / 16;  // 16-byte vectors of a lane
   const float inv = 1.0f / lt;
   const float lse = (m + log2f(lt)) * kLn2;
+  auto col = [&](int i) { return 16 * i + 8 * g; };
+  // The output rounded to the query type, columns col(i) .. col(i) + 7.
+  auto packed = [&](int i) {
+    const f32x16& o = oacc[i >> 1];
+    const int e = 8 * (i & 1);
+    u32x4 v;
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      const unsigned lo = pack2<T>(o[e + 2 * w] * inv, o[e + 2 * w + 1] * inv);
+      const unsigned hi = pack2<T>(o[e + 4 + 2 * w] * inv, o[e + 4 + 2 * w + 1] * inv);
+      const auto x = __builtin_amdgcn_permlane32_swap(lo, hi, false, false);
+      v[w] = x[0];
+      v[2 + w] = x[1];
+    }
+    return v;
+  };
 
   if constexpr (MODE == kModeHead) {
     // Head branch in the query type (the reference's head is the bf16 tensor its attention
     // kernel returns, recap/operator.py:366-370); the capture reads it back from here.
     uint16_t* orow = a.head_out + ((int64_t)bank * a.n_tokens + r) * D;
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int d0 = 32 * dt + 8 * q4 + 4 * g;
-        u32x2 v = {pack2<T>(oacc[dt][4 * q4] * inv, oacc[dt][4 * q4 + 1] * inv),
-                   pack2<T>(oacc[dt][4 * q4 + 2] * inv, oacc[dt][4 * q4 + 3] * inv)};
-        *reinterpret_cast<u32x2*>(orow + d0) = v;
-      }
+    for (int i = 0; i < NV; ++i) *reinterpret_cast<u32x4*>(orow + col(i)) = packed(i);
     if (g == 0) a.head_lse[(int64_t)bank * a.n_tokens + r] = lse;
     return;
   }
@@ -100,14 +125,7 @@ __device__ inline void store_rows(const AttnArgs& a, int bank, int b, int h, int
   uint16_t* orow = a.out + b * a.osB + h * a.osH + (int64_t)nat * a.osN;
   if constexpr (MODE == kModeDense) {
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int d0 = 32 * dt + 8 * q4 + 4 * g;
-        u32x2 v = {pack2<T>(oacc[dt][4 * q4] * inv, oacc[dt][4 * q4 + 1] * inv),
-                   pack2<T>(oacc[dt][4 * q4 + 2] * inv, oacc[dt][4 * q4 + 3] * inv)};
-        *reinterpret_cast<u32x2*>(orow + d0) = v;
-      }
+    for (int i = 0; i < NV; ++i) *reinterpret_cast<u32x4*>(orow + col(i)) = packed(i);
     if (g == 0) a.lse_native[(int64_t)bank * a.n_tokens + nat] = lse;
     return;
   }
@@ -118,9 +136,18 @@ __device__ inline void store_rows(const AttnArgs& a, int bank, int b, int h, int
   // .to(float32) at recap/kernels/detail_cache.py:228-234).
   if (r < a.rows) {
     const int64_t ri = (int64_t)bank * a.rows + r;
+    const uint16_t* gorow = a.go + ri * D;
+    const uint16_t* drow = a.det + ri * D;
+    u32x4 gv[NV], dv[NV];
     const float glv = a.gl[ri], dlv = a.dl[ri];
-    const float admit = a.use_override ? a.alpha_override
-                                       : expf(-fabsf(glv - a.glref[ri] - a.center[bank]));
+    float move = 0.0f;
+    if (!a.use_override) move = glv - a.glref[ri] - a.center[bank];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) gv[i] = *reinterpret_cast<const u32x4*>(gorow + col(i));
+#pragma unroll
+    for (int i = 0; i < NV; ++i) dv[i] = *reinterpret_cast<const u32x4*>(drow + col(i));
+    asm volatile("" ::: "memory");  // all of them before the first store
+    const float admit = a.use_override ? a.alpha_override : expf(-fabsf(move));
     const float cl = glv + dlv;
     const float tc = fmaxf(glv, cl);
     const float sm = (1.0f - admit) * expf(glv - tc);
@@ -133,43 +160,105 @@ __device__ inline void store_rows(const AttnArgs& a, int bank, int b, int h, int
     const float den2 = fmaxf(wh + wt, 1.0e-30f);
     // One reciprocal per denominator and row instead of a division per element.
     const float rden = 1.0f / den, rden2 = 1.0f / den2;
-    const uint16_t* gorow = a.go + ri * D;
-    const uint16_t* drow = a.det + ri * D;
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
+    for (int i = 0; i < NV; ++i) {
+      const u32x4 hv = packed(i);
+      u32x4 v;
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int d0 = 32 * dt + 8 * q4 + 4 * g;
-        const u32x2 gw = *reinterpret_cast<const u32x2*>(gorow + d0);
-        const u32x2 dw = *reinterpret_cast<const u32x2*>(drow + d0);
-        const u32x2 hw = {pack2<T>(oacc[dt][4 * q4] * inv, oacc[dt][4 * q4 + 1] * inv),
-                          pack2<T>(oacc[dt][4 * q4 + 2] * inv, oacc[dt][4 * q4 + 3] * inv)};
-        float res[4];
+      for (int w = 0; w < 4; ++w) {
+        float res[2];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const unsigned gword = gw[e >> 1], dword = dw[e >> 1], hword = hw[e >> 1];
-          const float gov = T::to_f((uint16_t)((e & 1) ? gword >> 16 : gword & 0xffff));
-          const float detv = f16_to_f((uint16_t)((e & 1) ? dword >> 16 : dword & 0xffff));
-          const float ohv = T::to_f((uint16_t)((e & 1) ? hword >> 16 : hword & 0xffff));
+        for (int e = 0; e < 2; ++e) {
+          const float gov = T::to_f((uint16_t)(e ? gv[i][w] >> 16 : gv[i][w] & 0xffff));
+          const float detv = f16_to_f((uint16_t)(e ? dv[i][w] >> 16 : dv[i][w] & 0xffff));
+          const float ohv = T::to_f((uint16_t)(e ? hv[w] >> 16 : hv[w] & 0xffff));
           const float to = (gov * sm + (gov + detv) * cm) * rden;
           res[e] = (ohv * wh + to * wt) * rden2;
         }
-        u32x2 v = {pack2<T>(res[0], res[1]), pack2<T>(res[2], res[3])};
-        *reinterpret_cast<u32x2*>(orow + d0) = v;
+        v[w] = pack2<T>(res[0], res[1]);
       }
+      *reinterpret_cast<u32x4*>(orow + col(i)) = v;
+    }
   } else {
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int d0 = 32 * dt + 8 * q4 + 4 * g;
-        u32x2 v = {pack2<T>(oacc[dt][4 * q4] * inv, oacc[dt][4 * q4 + 1] * inv),
-                   pack2<T>(oacc[dt][4 * q4 + 2] * inv, oacc[dt][4 * q4 + 3] * inv)};
-        *reinterpret_cast<u32x2*>(orow + d0) = v;
-      }
+    for (int i = 0; i < NV; ++i) *reinterpret_cast<u32x4*>(orow + col(i)) = packed(i);
   }
 }
 
+// The segments of a long row: each one's state (O^T, running max, row sum) goes to the
+// workspace, and the last one to arrive combines them all, in segment order, so the result
+// does not depend on which one that is.  True for the workgroup that then holds the row's
+// state.  The segments run on different XCDs, whose L2 caches are not coherent within a
+// launch: the state is written and read with the SC1 bit (agent scope), past those caches, and
+// every store has been acknowledged (vmcnt) before its segment is counted.
+template <int D>
+__device__ inline bool merge_segments(const AttnArgs& a, int item, int seg, int nseg, int* shared,
+                                      f32x16 (&oacc)[D / 32], float& m, float& lt) {
+  static_assert(kGroups == 1, "one query group per wave");
+  constexpr int NDT = D / 32;
+  constexpr int kAgent = 16;             // SC1
+  constexpr int kVec = 16 * kThreads;    // bytes of one 16-byte vector of every thread
+  constexpr int kState = 4 * NDT * kVec; // O^T of a segment; max and sum follow it
+  constexpr int kBytes = attn_part_words(D) * 8;
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));  // keeps the addresses below out of the registers of the walk
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(a.part + (int64_t)item * nseg * attn_part_words(D)), 0, nseg * kBytes, kBufferRsrcWord3);
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int e = 0; e < 16; e += 4) {
+      const f32x4 x = {oacc[dt][e], oacc[dt][e + 1], oacc[dt][e + 2], oacc[dt][e + 3]};
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), rs,
+                                             16 * t + (4 * dt + e / 4) * kVec, seg * kBytes, kAgent);
+    }
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, f32x2{m, lt}), rs, kState + 8 * t,
+                                        seg * kBytes, kAgent);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(kWaitVmLgkm0);
+  __syncthreads();
+  if (t == 0)
+    *shared = (int)__hip_atomic_fetch_add(a.tickets + item, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(*shared) != nseg - 1) return false;
+  float ms[kMaxSplit], ls[kMaxSplit];
+#pragma unroll
+  for (int s = 0; s < kMaxSplit; ++s) {
+    ms[s] = -INFINITY;
+    ls[s] = 0.0f;
+    if (s < nseg) {
+      const f32x2 x = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, kState + 8 * t, s * kBytes, kAgent));
+      ms[s] = x[0];
+      ls[s] = x[1];
+    }
+  }
+  float top = ms[0];
+#pragma unroll
+  for (int s = 1; s < kMaxSplit; ++s) top = fmaxf(top, ms[s]);
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) oacc[dt] = f32x16{};
+  m = top;
+  lt = 0.0f;
+#pragma unroll
+  for (int s = 0; s < kMaxSplit; ++s) {
+    if (s < nseg) {
+      // The whole state requested before its first use.
+      u32x4 x[4 * NDT];
+#pragma unroll
+      for (int i = 0; i < 4 * NDT; ++i)
+        x[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * t + i * kVec, s * kBytes, kAgent);
+      __builtin_amdgcn_sched_barrier(0);
+      const float w = ms[s] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms[s] - top);
+      lt = fmaf(w, ls[s], lt);
+#pragma unroll
+      for (int i = 0; i < 4 * NDT; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          oacc[i / 4][4 * (i % 4) + e] = fmaf(w, __uint_as_float(x[i][e]), oacc[i / 4][4 * (i % 4) + e]);
+    }
+  }
+  return true;
+}
 
 template <class T, int D, int MODE>
 __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
@@ -187,7 +276,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) char v_lds0[HALF];
   __shared__ __attribute__((aligned(16))) char v_lds1[HALF];
   __shared__ int list[MODE == kModeDense ? 1 : kMaxTiles];
-  __shared__ int scan[kThreads];
+  __shared__ int counts[kMaxTiles / 64];  // kept blocks per 64 blocks of the mask row
 
   const int t = threadIdx.x, lane = t & 63, g = lane >> 5, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -206,8 +295,24 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
   // next XCD that still has one; it stops when every queue is empty.  XCDs that run faster
   // then process the slower ones' last items instead of idling.  Every increment below an
   // XCD's count claims a distinct position, so each item is processed exactly once.
+  //
+  // In the masked modes each long row is `split` items, segments of its list of kept blocks:
+  // a long row alone takes as long as tb / keep of the others, which bounds a launch with few
+  // rounds of items (see attn_split).
   __shared__ int claimed;
-  const int n_items = a.banks * a.tb;
+  // The arguments that only one part of an item needs are read again there from the kernel's
+  // argument segment: kept over the walk they would take registers from it.
+  auto reread = []() -> const AttnArgs& {
+    typedef const __attribute__((address_space(4))) AttnArgs KernelArgs;
+    KernelArgs* args = (KernelArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    return *(const AttnArgs*)args;
+  };
+  constexpr bool kSplits = MODE == kModeHead || MODE == kModeMerge;
+  const int split = kSplits ? a.split : 1;
+  const int nlong = a.tb - a.ds, nshort = a.ds;
+  const int n_long_items = a.banks * nlong * split;
+  const int n_items = n_long_items + a.banks * nshort;
   const bool persistent = a.queue != nullptr;
   for (int round = 0;; ++round) {
   int pos = blockIdx.x;
@@ -229,12 +334,13 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
   } else if (round > 0) {
     break;
   }
-  const int nlong = a.tb - a.ds, nshort = a.ds;
-  const int n_long_items = a.banks * nlong;
-  int bank, qt;
+  int bank, qt, seg = 0, nseg = 1;
   if (pos < n_long_items) {
-    bank = pos / nlong;
-    qt = a.ds + pos % nlong;
+    const int li = pos / split;
+    bank = li / nlong;
+    qt = a.ds + li % nlong;
+    seg = pos % split;
+    nseg = split;
   } else {
     const int lin = xcd_runs(pos - n_long_items, n_items - n_long_items, 64);
     bank = lin / nshort;
@@ -242,38 +348,90 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
   }
   const int b = bank / a.heads, h = bank % a.heads;
 
-  int nkeep = a.tb;
+  const AttnArgs& early = reread();
+  // Query group q of this wave: rows 32 q .. 32 q + 31 of the wave's kRowsPerWave.  The row
+  // map, the mask row and the Q rows are all requested before the first of them is used.
+  int row[kGroups], nat[kGroups];
+  bool valid[kGroups];
+#pragma unroll
+  for (int q = 0; q < kGroups; ++q) {
+    row[q] = qt * kBlock + wave * kRowsPerWave + 32 * q + l32;
+    valid[q] = row[q] < a.n_tokens;
+    nat[q] = valid[q] ? early.rowmap[row[q]] : 0;
+  }
+  // A copy of the thread index that the compiler cannot see through: what is derived from it
+  // is computed per item instead of being kept in registers over all items.
+  int tt = t;
+  asm volatile("" : "+v"(tt));
+  constexpr int kChunks = MODE == kModeDense ? 1 : kMaxTiles / kThreads;
+  const int nchunks = (a.tb + kThreads - 1) / kThreads;
+  uint8_t cell[kChunks];
+  bool lead = false;
   if constexpr (MODE != kModeDense) {
-    // Kept blocks in ascending order; in dense-head mode the other blocks follow them.
-    const uint8_t* mrow = a.kmask + ((int64_t)bank * a.tb + qt) * a.tb;
-    const int per = (a.tb + kThreads - 1) / kThreads;
-    const int j0 = min(t * per, a.tb), j1 = min(j0 + per, a.tb);
-    int cnt = 0;
-    for (int j = j0; j < j1; ++j) cnt += mrow[j] != 0;
-    scan[t] = cnt;
-    __syncthreads();
-    for (int off = 1; off < kThreads; off <<= 1) {
-      const int v = t >= off ? scan[t - off] : 0;
-      __syncthreads();
-      scan[t] += v;
-      __syncthreads();
-    }
-    int pos = scan[t] - cnt;
-    nkeep = __builtin_amdgcn_readfirstlane(scan[kThreads - 1]);
-    int npos = nkeep + (j0 - pos);  // blocks not kept before this thread's range
+    const uint8_t* mrow = early.kmask + ((int64_t)bank * a.tb + qt) * a.tb;
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i)
+      if (i < nchunks) cell[i] = mrow[min(kThreads * i + tt, a.tb - 1)];
     // A kept ragged last block goes first, so its masked steps open the walk (in dense-head
     // mode the blocks that are not kept follow the kept ones, and the ragged block would
     // otherwise fall in the middle); every masked mode uses the same order.
-    const bool lead = (a.n_tokens % kBlock) != 0 && mrow[a.tb - 1] != 0;
-    for (int j = j0; j < j1; ++j) {
-      if (mrow[j]) {
-        list[lead ? (j == a.tb - 1 ? 0 : pos + 1) : pos] = j;
-        ++pos;
-      } else if (MODE == kModeDenseHead) {
-        list[npos++] = j;
+    lead = (a.n_tokens % kBlock) != 0 && mrow[a.tb - 1] != 0;
+  }
+  u32x4 qreg[kGroups][NS];
+#pragma unroll
+  for (int q = 0; q < kGroups; ++q) {
+    const uint16_t* qrow = early.q + b * early.qsB + h * early.qsH + (int64_t)nat[q] * early.qsN;
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      qreg[q][s] = valid[q] ? *reinterpret_cast<const u32x4*>(qrow + 16 * s + 8 * g)
+                            : u32x4{0u, 0u, 0u, 0u};
+  }
+
+  int nkeep = a.tb, first = 0;  // blocks of this item's walk: list[first ..]
+  if constexpr (MODE != kModeDense) {
+    // Kept blocks in ascending order; in dense-head mode the other blocks follow them.  Block
+    // j's place is the number of kept blocks before it: the counts of the earlier groups of
+    // 64 blocks, scanned by every wave for itself, plus the kept lanes below it in its
+    // ballot.  Two barriers a row (a scan over the 256 threads took 18).
+    const int ln = tt & 63;
+    unsigned kept = 0;
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i)
+      if (i < nchunks) {
+        const bool on = kThreads * i + tt < a.tb && cell[i] != 0;
+        const unsigned long long bal = __ballot(on);
+        kept |= (unsigned)on << i;
+        if (ln == 0) counts[kThreads / 64 * i + wave] = (int)__popcll(bal);
+      }
+    lds_barrier();
+    const int own = ln < kThreads / 64 * nchunks ? counts[ln] : 0;
+    int upto = own;  // inclusive
+#pragma unroll
+    for (int off = 1; off < kMaxTiles / 64; off <<= 1) {
+      const int u = __shfl_up(upto, off, 64);
+      if (ln >= off) upto += u;
+    }
+    nkeep = __builtin_amdgcn_readlane(upto, kMaxTiles / 64 - 1);
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i)
+      if (i < nchunks) {
+        const bool on = (kept >> i) & 1u;
+        const unsigned long long bal = __ballot(on);
+        const int j = kThreads * i + tt;
+        const int before = __shfl(upto - own, kThreads / 64 * i + wave, 64) +
+                           (int)__popcll(bal & ((1ull << ln) - 1ull));
+        if (on)
+          list[lead ? (j == a.tb - 1 ? 0 : before + 1) : before] = j;
+        else if (MODE == kModeDenseHead && j < a.tb)
+          list[nkeep + (j - before)] = j;
+      }
+    lds_barrier();
+    if constexpr (kSplits) {
+      if (nseg > 1) {
+        first = nkeep * seg / nseg;
+        nkeep = nkeep * (seg + 1) / nseg - first;
       }
     }
-    __syncthreads();
   }
   const int nsub = MODE == kModeDenseHead ? 2 * a.tb : 2 * nkeep;  // 64-key sub-tiles
 
@@ -283,11 +441,11 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
   // lane order) over this bank's images, whose byte size bounds the buffer resource.
   const int bank_bytes = a.tb * G::kTileBytes;
   const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(a.kp + (int64_t)bank * a.tb * G::kTileElems), 0, bank_bytes, kBufferRsrcWord3);
+      (void*)(early.kp + (int64_t)bank * a.tb * G::kTileElems), 0, bank_bytes, kBufferRsrcWord3);
   const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(a.vp + (int64_t)bank * a.tb * G::kTileElems), 0, bank_bytes, kBufferRsrcWord3);
+      (void*)(early.vp + (int64_t)bank * a.tb * G::kTileElems), 0, bank_bytes, kBufferRsrcWord3);
   auto image = [&](int it) {  // byte offset of sub-tile `it` within the bank's images
-    const int j = MODE == kModeDense ? (it >> 1) : list[it >> 1];
+    const int j = MODE == kModeDense ? (it >> 1) : list[first + (it >> 1)];
     return __builtin_amdgcn_readfirstlane(j * G::kTileBytes + (it & 1) * HALF);
   };
   auto copy = [&](__amdgpu_buffer_rsrc_t rs, int off, char* dst) {
@@ -298,29 +456,11 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
           16 * kThreads * i + 16 * t, off, 0, 0);
   };
 
-  // Query group q of this wave: rows 32 q .. 32 q + 31 of the wave's kRowsPerWave.
-  int row[kGroups], nat[kGroups];
-  bool valid[kGroups];
-#pragma unroll
-  for (int q = 0; q < kGroups; ++q) {
-    row[q] = qt * kBlock + wave * kRowsPerWave + 32 * q + l32;
-    valid[q] = row[q] < a.n_tokens;
-    nat[q] = valid[q] ? a.rowmap[row[q]] : 0;
-  }
   if (nsub > 0) {
     copy(krs, image(0), k_lds0);
     copy(vrs, image(0), v_lds0);
   }
   if (nsub > 1) copy(krs, image(1), k_lds1);
-  u32x4 qreg[kGroups][NS];
-#pragma unroll
-  for (int q = 0; q < kGroups; ++q) {
-    const uint16_t* qrow = a.q + b * a.qsB + h * a.qsH + (int64_t)nat[q] * a.qsN;
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-      qreg[q][s] = valid[q] ? *reinterpret_cast<const u32x4*>(qrow + 16 * s + 8 * g)
-                            : u32x4{0u, 0u, 0u, 0u};
-  }
   tile_barrier();
 
   float m[kGroups], mraw[kGroups], lsum[kGroups];
@@ -534,7 +674,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
 
   // True when sub-tile `it` of the list lies in the ragged last block.
   auto ragged_at = [&](int it) {
-    const int j = MODE == kModeDense ? (it >> 1) : __builtin_amdgcn_readfirstlane(list[it >> 1]);
+    const int j = MODE == kModeDense ? (it >> 1) : __builtin_amdgcn_readfirstlane(list[first + (it >> 1)]);
     return ragged && j == a.tb - 1;
   };
   f32x16 sa[kGroups][2], sb[kGroups][2];
@@ -576,13 +716,45 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
   }
 
   constexpr int kStore = MODE == kModeDenseHead ? kModeDense : MODE;
+  const AttnArgs& late = reread();
+  bool stores = true;
+  float lt[kGroups];
+#pragma unroll
+  for (int q = 0; q < kGroups; ++q)
+    lt[q] = pair_sum(lsum[q]);  // lanes l and l ^ 32 share one row: both valid or not
+  if constexpr (kSplits) {
+    if (nseg > 1) stores = merge_segments<D>(late, bank * nlong + (qt - a.ds), seg, nseg, &claimed, oacc[0], m[0], lt[0]);
+  }
+  int lane_row = l32;
+  asm volatile("" : "+v"(lane_row));  // the row numbers are computed again, not kept
 #pragma unroll
   for (int q = 0; q < kGroups; ++q) {
-    const float lt = pair_sum(lsum[q]);  // lanes l and l ^ 32 share one row: both valid or not
-    if (valid[q]) store_rows<T, D, kStore>(a, bank, b, h, row[q], nat[q], g, oacc[q], m[q], lt);
+    const int r = qt * kBlock + wave * kRowsPerWave + 32 * q + lane_row;
+    if (r < a.n_tokens && stores)
+      store_rows<T, D, kStore>(late, bank, b, h, r, nat[q], g, oacc[q], m[q], lt[q]);
   }
   __syncthreads();  // every wave is done with the LDS slots, the list and `claimed`
   }  // items
+}
+
+// Segments of each long row (query blocks ds .. tb-1, dense) of a masked launch whose other
+// rows keep about `density` of their blocks.  A long row as one item takes its tb tiles
+// however idle the chip is, so it is cut until a segment is no longer than the other items, or
+// than half of the work there is for each of the 512 workgroups, and not below 16 tiles (a
+// segment's state costs about two tiles to store and combine); and not so far that items which
+// fit one round of the 512 need a second.  Attention kernel, 1 segment -> this rule: 101 -> 73 us
+// at 12 banks of 38 blocks (2 segments; 3: 80, 6: 73), 203 -> 178 us at 12 of 61 (3; 6: 199),
+// 333 -> 275 us at 8 of 125 (4; 6: 276); no change at 12 of 256 (2).  It depends on the layer's
+// sizes only, so that every group of its heads is cut alike.
+int attn_split(int64_t banks, int64_t tb, int64_t ds, double density) {
+  if (ds >= tb) return 1;
+  const double longs = (double)(tb - ds), other = density * (double)tb + longs + 1.0;
+  const double share = (double)banks * ((double)ds * other + longs * (double)tb) / 512.0;
+  const double segment = std::max(16.0, std::max(other, 0.5 * share));
+  int split = (int)std::min<double>(kMaxSplit, std::max(1.0, std::ceil((double)tb / segment)));
+  while (split > 2 && banks * (ds + (tb - ds) * split) > 512 && banks * (ds + (tb - ds) * 2) <= 512)
+    --split;
+  return split;
 }
 
 // Workgroups of a persistent launch: two per CU (the attention kernel's occupancy), no
@@ -598,7 +770,8 @@ static int persistent_grid(int items) {
 
 template <class T, int D>
 static hipError_t launch_attention(const AttnArgs& a, int mode, hipStream_t s) {
-  const int items = a.banks * a.tb;
+  const bool splits = mode == kModeHead || mode == kModeMerge;
+  const int items = a.banks * (a.ds + (a.tb - a.ds) * (splits ? a.split : 1));
   const dim3 grid((unsigned)(a.queue != nullptr ? persistent_grid(items) : items)), block(kThreads);
   switch (mode) {
     case kModeHead: hipLaunchKernelGGL((attention_kernel<T, D, kModeHead>), grid, block, 0, s, a); break;

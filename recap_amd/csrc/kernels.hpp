@@ -107,7 +107,14 @@ struct AttnArgs {
   int rows; const uint16_t* go; const float* gl; const uint16_t* det; const float* dl;
   const float* glref; const float* center; float alpha_override; int use_override;
   unsigned* queue;   // kQueueWords zeroed words: per-XCD claim counters, or null (static)
+  // Head and merge modes: segments of a long row (1: none), their states (attn_part_words(D)
+  // 8-byte words each) and one zeroed arrival counter per long row.
+  int split = 1; unsigned long long* part; unsigned* tickets;
 };
+constexpr int kMaxSplit = 8;
+int attn_split(int64_t banks, int64_t tb, int64_t ds, double density);
+// 8-byte words of one segment's state: O^T, running max and row sum of 256 threads.
+__host__ __device__ constexpr int attn_part_words(int dim) { return (dim / 4 + 1) * 256; }
 hipError_t run_attention(const AttnArgs& a, int dtype, int dim, int mode, hipStream_t s);
 // Claim counters of the attention launch's work queues: one per XCD, 128 bytes apart.
 constexpr int kQueueStride = 32;

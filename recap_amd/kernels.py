@@ -44,6 +44,9 @@ class Geometry:
     # Video blocks per closure-statistics workgroup, fixed for a whole layer (the partial
     # sums, and so the rounding, depend on it); None: chosen from the call's banks.
     closure_group: int | None = None
+    # Segments of each long query row of the masked attention, fixed for a whole layer like
+    # the group above; None: chosen from the call's banks.
+    attn_split: int | None = None
 
     @property
     def nb(self) -> int:
@@ -350,10 +353,26 @@ def block_sparse_attn(q: torch.Tensor, kv: PackedKV, rowmap: torch.Tensor,
     kernel_mask = kernel_mask.contiguous()
     out = torch.empty(b * h, n, d, dtype=q.dtype, device=q.device)
     lse = torch.empty(b * h, n, dtype=torch.float32, device=q.device)
-    call("recap_block_sparse_attn", *_qkv_args(q), kv.k_tiles.data_ptr(), kv.vt_tiles.data_ptr(),
-         rowmap.data_ptr(), kernel_mask.data_ptr(), n, float(scale), out.data_ptr(),
-         lse.data_ptr(), _stream())
+    split, work = _attn_workspace(q, geo)
+    call("recap_block_sparse_attn_ws", *_qkv_args(q), kv.k_tiles.data_ptr(),
+         kv.vt_tiles.data_ptr(), rowmap.data_ptr(), kernel_mask.data_ptr(), n, geo.n_video,
+         float(scale), out.data_ptr(), lse.data_ptr(), split, 1, work.data_ptr(), work.numel(),
+         _stream())
     return out, lse
+
+
+def attn_split(banks: int, geo: Geometry, density: float = 0.25) -> int:
+    """Segments of each long query row for a layer of `banks` heads whose other rows keep about
+    `density` of their blocks."""
+    return int(_lib.load().recap_attn_split(banks, geo.n_tokens, geo.n_video, float(density)))
+
+
+def _attn_workspace(q: torch.Tensor, geo: Geometry) -> tuple[int, torch.Tensor]:
+    """(split, workspace) of a masked attention launch."""
+    b, h, _, d = q.shape
+    split = geo.attn_split or attn_split(b * h, geo)
+    size = int(_lib.load().recap_attn_workspace_size(b * h, d, geo.n_tokens, geo.n_video, split))
+    return split, torch.empty(size, dtype=torch.uint8, device=q.device)
 
 
 def dense_attn(q: torch.Tensor, kv: PackedKV, rowmap: torch.Tensor, scale: float,
@@ -414,11 +433,12 @@ def sparse_merge_attn(q: torch.Tensor, kv: PackedKV, rowmap: torch.Tensor,
     if out is None:
         out = torch.empty(b, h, n, d, dtype=q.dtype, device=q.device)
     alpha = -1.0 if alpha_override is None else float(alpha_override)
-    call("recap_sparse_merge_attn", *_qkv_args(q), kv.k_tiles.data_ptr(),
+    split, work = _attn_workspace(q, geo)
+    call("recap_sparse_merge_attn_ws", *_qkv_args(q), kv.k_tiles.data_ptr(),
          kv.vt_tiles.data_ptr(), rowmap.data_ptr(), kernel_mask.data_ptr(), n, geo.n_video,
          float(scale), _p(go), _p(gl), _p(det), _p(dl), _p(glref), _p(center), alpha,
-         out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
-         _p(_work_queue(q.device, balance)), _stream())
+         out.data_ptr(), out.stride(0), out.stride(1), out.stride(2), split, int(balance),
+         work.data_ptr(), work.numel(), _stream())
     return out
 
 

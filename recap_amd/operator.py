@@ -275,8 +275,10 @@ class Operator:
         self.layout._check(query)
         banks = query.shape[0] * query.shape[1]
         nb = -(-self.layout.video_tokens // K.BLOCK)
-        return K.Geometry(n_tokens=query.shape[-2], n_video=self.layout.video_tokens,
-                          closure_group=K.closure_group(banks, nb))
+        geo = K.Geometry(n_tokens=query.shape[-2], n_video=self.layout.video_tokens,
+                         closure_group=K.closure_group(banks, nb))
+        return dataclasses.replace(
+            geo, attn_split=K.attn_split(banks, geo, self.config.head_density))
 
     @torch.no_grad()
     def attend(self, layer_index: int, query: torch.Tensor, key: torch.Tensor,

@@ -231,6 +231,51 @@ def test_attention_modes_short_and_ragged(cuda, n, d, keep_last):
         assert m < 2e-3, m
 
 
+@pytest.mark.parametrize("n,n_video,d,dtype", [
+    (700, 600, 128, torch.bfloat16),    # ragged video block shared with text, ragged last block
+    (700, 640, 64, torch.bfloat16),     # whole video blocks beside text
+    (389, 389, 128, torch.float16),     # video only, ragged: one long row
+    (4300, 4200, 64, torch.float16)])   # more blocks than one ballot covers
+def test_split_long_rows(cuda, n, n_video, d, dtype):
+    """Long rows cut into segments (two, three and eight, more than a short row has blocks):
+    the other rows bit for bit those of one segment, every row within the bar of the oracle,
+    the same bits on every run and without claim queues, in head and merge modes."""
+    g = torch.Generator().manual_seed(n + d)
+    banks, tb = 2, -(-n // 128)
+    q, k, v = (torch.randn(1, banks, n, d, generator=g).to(dtype) for _ in range(3))
+    first = n_video // 128
+    kmask = torch.rand(banks, tb, tb, generator=g) > 0.6
+    kmask[:, torch.arange(tb), torch.arange(tb)] = True
+    kmask[:, first:] = True
+    kmask[0, -1, : tb - 1] = False   # a long row that keeps one block: segments without work
+    ql, kl, vl = (x[0].float() for x in (q, k, v))
+    ref, ref_lse = O.block_sparse_attention(ql, kl, vl, kmask, scale_for(d))
+    q, k, v, kmask = (x.to(cuda) for x in (q, k, v, kmask))
+    rowmap = torch.arange(n, dtype=torch.int32, device=cuda)
+    rows = 128 * first
+    gl = torch.randn(banks, rows, generator=g).to(cuda)
+    go = torch.randn(banks, rows, d, generator=g).to(cuda, dtype)
+    det = torch.randn(banks, rows, d, generator=g).to(cuda, torch.float16)
+    dl = torch.randn(banks, rows, generator=g).to(cuda)
+    center = torch.zeros(banks, device=cuda)
+    kv = K.kv_pack(k, v, rowmap, K.Geometry(n, n_video))
+    outs = {}
+    for split in (1, 2, 3, 8):
+        geo = K.Geometry(n, n_video, attn_split=split)
+        print(f"case n={n} d={d} split={split}", flush=True)
+        head, lse = K.block_sparse_attn(q, kv, rowmap, kmask, geo, scale_for(d))
+        merge = [K.sparse_merge_attn(q, kv, rowmap, kmask, geo, scale_for(d), go, gl, det, dl,
+                                     gl, center, balance=balance)[0]
+                 for balance in (True, True, False)]
+        assert torch.equal(merge[0], merge[1]) and torch.equal(merge[0], merge[2])
+        assert_parity(head.cpu().float(), ref, f"split {split}", dtype=dtype)
+        assert float((lse.cpu() - ref_lse).abs().max()) < 2e-3
+        assert torch.equal(merge[0][:, rows:], head[:, rows:])
+        outs[split] = head[:, :rows], lse[:, :rows], merge[0][:, :rows]
+        for a, b in zip(outs[split], outs[1]):
+            assert torch.equal(a, b), split
+
+
 @pytest.mark.parametrize("d", [64, 128])
 def test_attention_running_max_jumps(cuda, d):
     """Keys of each 64-key sub-tile scaled by factors from 0.1 to 80, so that a row's scores
