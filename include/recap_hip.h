@@ -281,6 +281,33 @@ int recap_sparse_merge_attn_ws(const void* q, int dtype, int64_t batch, int64_t 
                                int64_t out_stride_n, int64_t split, int balance,
                                void* workspace, int64_t workspace_bytes, void* stream);
 
+/* A whole corrected sparse call of a layer with a frozen basis, as five launches on `stream`:
+ * recap_kv_pack, recap_closure_stats (ROT | CVK, `group` blocks a workgroup), the C_vk and
+ * coarse tables in one launch that also zeroes the attention counters, recap_coarse_tail and
+ * recap_sparse_merge_attn_ws, whose waves take the drift centre from the coarse tail's partial
+ * sums.  Outputs are those of the separate calls, bit for bit.  `u_hi_t`, `u_lo_t` and `u_t`
+ * are the tables of recap_basis_tables; `det`, `dl`, `glref`, `partition` and `kernel_mask`
+ * the layer's bank; the workspace (recap_sparse_call_workspace_size bytes, 16-byte aligned)
+ * needs no contents and keeps none.  `stage_events`, unless NULL, holds five hipEvent_t
+ * recorded before the first launch and after the pack, tables, coarse and attention launches.
+ * Nothing is launched when an argument is rejected.
+ * Replaces Operator._sparse, recap/operator.py:477-527. */
+int64_t recap_sparse_call_workspace_size(int dtype, int64_t banks, int64_t dim, int64_t n_tokens,
+                                         int64_t n_video, int64_t group, int64_t rank,
+                                         int64_t split);
+int recap_sparse_call(const void* q, const void* k, const void* v, int dtype, int64_t batch,
+                      int64_t heads, int64_t dim, int64_t q_stride_b, int64_t q_stride_h,
+                      int64_t q_stride_n, int64_t k_stride_b, int64_t k_stride_h,
+                      int64_t k_stride_n, int64_t v_stride_b, int64_t v_stride_h,
+                      int64_t v_stride_n, const int32_t* rowmap, int64_t n_tokens,
+                      int64_t n_video, float scale, float theta, int64_t rank, int64_t group,
+                      const void* u_hi_t, const void* u_lo_t, const void* u_t,
+                      const uint8_t* partition, const uint8_t* kernel_mask, const void* det,
+                      const float* dl, const float* glref, float alpha_override, void* out,
+                      int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_n,
+                      int64_t split, void* const* stage_events, void* workspace,
+                      int64_t workspace_bytes, void* stream);
+
 /* Stage 4 ------------------------------------------------------------------------------ */
 
 /* Number of (err2, ref2) partial pairs recap_refresh_capture writes. */

@@ -348,8 +348,11 @@ int recap_coarse_tables(const float* variance, const float* k_means, const float
   CHECK(check_common(dtype, dim));
   REQUIRE(variance && k_means && v_means && w && kbar && vbar, "NULL pointer");
   REQUIRE(banks >= 1 && n_blocks >= 1 && rank >= 0, "bad sizes");
-  TablesArgs a{variance, k_means, v_means, (int)banks, (int)n_blocks, (int)dim, (int)rank,
-               static_cast<uint16_t*>(w), static_cast<uint16_t*>(kbar), static_cast<uint16_t*>(vbar)};
+  TablesArgs a{};
+  a.var = variance; a.kmean = k_means; a.vmean = v_means;
+  a.banks = (int)banks; a.nb = (int)n_blocks; a.dim = (int)dim; a.rank = (int)rank;
+  a.w_t = static_cast<uint16_t*>(w); a.kbar_t = static_cast<uint16_t*>(kbar);
+  a.vbar_t = static_cast<uint16_t*>(vbar);
   return hip_status(run_tables(a, dtype, as_stream(stream)), "coarse_tables launch");
 }
 
@@ -581,7 +584,8 @@ static int merge_args(const void* q, int dtype, int64_t batch, int64_t heads, in
   REQUIRE(kernel_mask != nullptr, "kernel_mask is NULL");
   if (a.rows > 0) {
     REQUIRE(go && gl && det && dl && aligned16(go) && aligned16(det), "merge inputs go/gl/det/dl");
-    REQUIRE(alpha_override >= 0.0f || (glref && center), "drift weight needs glref and center");
+    REQUIRE(alpha_override >= 0.0f || (glref && (center || a.drift_part)),
+            "drift weight needs glref and center");
   }
   a.kmask = kernel_mask;
   CHECK(set_scale(a, scale));
@@ -626,6 +630,125 @@ int recap_sparse_merge_attn_ws(const void* q, int dtype, int64_t batch, int64_t 
                    alpha_override, out, out_stride_b, out_stride_h, out_stride_n, a));
   CHECK(set_workspace(a, dim, split, balance, workspace, workspace_bytes, as_stream(stream)));
   return hip_status(run_attention(a, dtype, (int)dim, kModeMerge, as_stream(stream)), "attention launch");
+}
+
+// Workspace of recap_sparse_call: byte offsets of its parts.
+struct SparseSpace {
+  int64_t kt, vt, km, vm, var, cvk_t, w, kbar, vbar, cvk_part, go, gl, drift, attn, attn_bytes, bytes;
+};
+
+static SparseSpace sparse_space(int dtype, int64_t banks, int64_t dim, const Geom& g, int64_t n_video,
+                                int64_t group, int64_t rank, int64_t split) {
+  SparseSpace w;
+  int64_t at = 0;
+  auto take = [&](int64_t bytes) { const int64_t o = at; at += align256(bytes); return o; };
+  const int64_t padded = (g.nb + kCoarseSlots - 1) / kCoarseSlots * kCoarseSlots;
+  const int64_t groups = (g.nb + group - 1) / group;
+  w.kt = take(banks * g.tb * kBlock * dim * 2);
+  w.vt = take(banks * g.tb * kBlock * dim * 2);
+  w.km = take(banks * g.nb * dim * 4);
+  w.vm = take(banks * g.nb * dim * 4);
+  w.var = take(banks * g.nb * dim * 4);
+  w.cvk_t = take(banks * dim * dim * 2);
+  w.w = take(banks * padded * (coarse_folded(dtype, (int)dim, (int)rank) ? kFoldCols : dim) * 2);
+  w.kbar = take(banks * padded * dim * 2);
+  w.vbar = take(banks * padded * dim * 2);
+  // The C_vk partials are read before the coarse output is written.
+  w.cvk_part = w.go = take(std::max(banks * groups * dim * dim * 4, banks * g.rows * dim * 2));
+  w.gl = take(banks * g.rows * 4);
+  w.drift = take(banks * (g.rows / kBlock) * 4);
+  w.attn_bytes = attn_space(banks, dim, g.tb - first_long(g, n_video), split).bytes;
+  w.attn = take(w.attn_bytes);
+  w.bytes = at;
+  return w;
+}
+
+int64_t recap_sparse_call_workspace_size(int dtype, int64_t banks, int64_t dim, int64_t n_tokens,
+                                         int64_t n_video, int64_t group, int64_t rank,
+                                         int64_t split) {
+  if (check_common(dtype, dim) != RECAP_OK || check_tokens(n_tokens, n_video) != RECAP_OK ||
+      banks < 1 || group < 1 || rank < 0 || split < 1 || split > kMaxSplit)
+    return -1;
+  return sparse_space(dtype, banks, dim, geometry(n_tokens, n_video), n_video, group, rank, split).bytes;
+}
+
+int recap_sparse_call(const void* q, const void* k, const void* v, int dtype, int64_t batch,
+                      int64_t heads, int64_t dim, int64_t q_stride_b, int64_t q_stride_h,
+                      int64_t q_stride_n, int64_t k_stride_b, int64_t k_stride_h,
+                      int64_t k_stride_n, int64_t v_stride_b, int64_t v_stride_h,
+                      int64_t v_stride_n, const int32_t* rowmap, int64_t n_tokens,
+                      int64_t n_video, float scale, float theta, int64_t rank, int64_t group,
+                      const void* u_hi_t, const void* u_lo_t, const void* u_t,
+                      const uint8_t* partition, const uint8_t* kernel_mask, const void* det,
+                      const float* dl, const float* glref, float alpha_override, void* out,
+                      int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_n,
+                      int64_t split, void* const* stage_events, void* workspace,
+                      int64_t workspace_bytes, void* stream) {
+  // Every check of the five launches is made before the first of them.
+  CHECK(check_common(dtype, dim));
+  CHECK(check_tokens(n_tokens, n_video));
+  CHECK(check_qkv("k", k, batch, heads, k_stride_b, k_stride_h, k_stride_n));
+  CHECK(check_qkv("v", v, batch, heads, v_stride_b, v_stride_h, v_stride_n));
+  REQUIRE(rowmap && partition && u_hi_t && u_lo_t && u_t, "NULL pointer");
+  REQUIRE(aligned16(u_hi_t) && aligned16(u_lo_t) && aligned16(u_t), "tables must be 16-byte aligned");
+  REQUIRE(theta >= 0.0f, "theta must be non-negative");
+  REQUIRE(rank >= 0 && rank <= dim, "rank %lld outside [0, dim]", (long long)rank);
+  REQUIRE(group >= 1, "bad group");
+  REQUIRE(split >= 1 && split <= kMaxSplit, "split %lld outside 1..%d", (long long)split, kMaxSplit);
+  REQUIRE(workspace != nullptr && aligned16(workspace), "workspace must be non-NULL and 16-byte aligned");
+  const Geom g = geometry(n_tokens, n_video);
+  REQUIRE(g.nb <= 4096, "too many video blocks (%lld > 4096)", (long long)g.nb);
+  REQUIRE(batch >= 1 && heads >= 1, "bad batch/heads");
+  const int64_t banks = batch * heads;
+  const SparseSpace w = sparse_space(dtype, banks, dim, g, n_video, group, rank, split);
+  REQUIRE(workspace_bytes >= w.bytes, "workspace of %lld bytes, need %lld",
+          (long long)workspace_bytes, (long long)w.bytes);
+  char* base = static_cast<char*>(workspace);
+  auto f32 = [&](int64_t o) { return reinterpret_cast<float*>(base + o); };
+  hipStream_t s = as_stream(stream);
+  AttnArgs a{};
+  a.drift_part = f32(w.drift);
+  CHECK(merge_args(q, dtype, batch, heads, dim, q_stride_b, q_stride_h, q_stride_n, base + w.kt,
+                   base + w.vt, rowmap, kernel_mask, n_tokens, n_video, scale, base + w.go,
+                   f32(w.gl), det, dl, glref, nullptr, alpha_override, out, out_stride_b,
+                   out_stride_h, out_stride_n, a));
+  unsigned* words = reinterpret_cast<unsigned*>(base + w.attn);
+  const AttnSpace space = attn_space(banks, dim, a.tb - a.ds, split);
+  a.queue = words;
+  a.split = a.tb > a.ds ? (int)split : 1;
+  a.tickets = words + kQueueWords;
+  a.part = reinterpret_cast<unsigned long long*>(words + space.counters);
+
+  auto mark = [&](int i) -> int {
+    if (stage_events == nullptr) return RECAP_OK;
+    return hip_status(hipEventRecord(static_cast<hipEvent_t>(stage_events[i]), s), "stage event");
+  };
+  CHECK(mark(0));
+  CHECK(recap_kv_pack(k, v, dtype, batch, heads, dim, k_stride_b, k_stride_h, k_stride_n,
+                      v_stride_b, v_stride_h, v_stride_n, rowmap, n_tokens, n_video, base + w.kt,
+                      base + w.vt, f32(w.km), f32(w.vm), stream));
+  CHECK(mark(1));
+  CHECK(recap_closure_stats(base + w.kt, base + w.vt, f32(w.km), dtype, u_hi_t, u_lo_t, banks, dim,
+                            n_tokens, n_video, group, RECAP_CLOSURE_ROT | RECAP_CLOSURE_CVK,
+                            f32(w.var), f32(w.cvk_part), nullptr, stream));
+  TablesArgs t{};
+  t.var = f32(w.var); t.kmean = f32(w.km); t.vmean = f32(w.vm);
+  t.banks = (int)banks; t.nb = (int)g.nb; t.dim = (int)dim; t.rank = (int)rank;
+  t.w_t = reinterpret_cast<uint16_t*>(base + w.w);
+  t.kbar_t = reinterpret_cast<uint16_t*>(base + w.kbar);
+  t.vbar_t = reinterpret_cast<uint16_t*>(base + w.vbar);
+  t.cvk_part = f32(w.cvk_part); t.groups = (int)recap_closure_groups(n_video, group);
+  t.divisor = (float)n_video; t.cvk_t = reinterpret_cast<uint16_t*>(base + w.cvk_t);
+  t.zero = words; t.zero_words = (int)space.counters;
+  CHECK(hip_status(run_tables(t, dtype, s), "tables launch"));
+  CHECK(mark(2));
+  CHECK(recap_coarse_tail(q, dtype, batch, heads, dim, q_stride_b, q_stride_h, q_stride_n, rowmap,
+                          partition, base + w.kbar, base + w.vbar, base + w.w, u_t, base + w.cvk_t,
+                          n_tokens, n_video, scale, theta, rank, glref, base + w.go, f32(w.gl),
+                          f32(w.drift), stream));
+  CHECK(mark(3));
+  CHECK(hip_status(run_attention(a, dtype, (int)dim, kModeMerge, s), "attention launch"));
+  return mark(4);
 }
 
 int64_t recap_attn_queue_words(void) { return kQueueWords; }

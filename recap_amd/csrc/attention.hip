@@ -82,6 +82,22 @@ constexpr int kGroups = 1;
 constexpr int kRowsPerWave = 32 * kGroups;
 constexpr int kThreads = 64 * (kBlock / kRowsPerWave);
 
+// A bank's drift centre from the coarse tail's partial sums, in drift_center's order (256
+// threads' runs, then its halving tree), by one whole wave: a launch of its own less per call.
+__device__ inline float drift_centre(const float* part, int tiles, int rows) {
+  const int lane = threadIdx.x & 63, per = (tiles + 255) / 256;
+  float v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int t = lane + 64 * k;
+    v[k] = 0.0f;
+    for (int i = t * per; i < min((t + 1) * per, tiles); ++i) v[k] += part[i];
+  }
+  float x = (v[0] + v[2]) + (v[1] + v[3]);
+  for (int off = 32; off >= 1; off >>= 1) x += __shfl_down(x, off, 64);
+  return __uint_as_float((unsigned)__builtin_amdgcn_readfirstlane((int)__float_as_uint(x))) / (float)rows;
+}
+
 // Final normalisation and store of one query row per lane pair, in the layout of the kernel's
 // mode.  Lane (g, l32) holds columns 32 dt + 8 q4 + 4 g .. +3 of its row; one exchange of
 // packed words within the lane pair gives it 8 consecutive ones, 32 dt + 16 j + 8 g .., so that
@@ -141,7 +157,14 @@ __device__ inline void store_rows(const AttnArgs& a, int bank, int b, int h, int
     u32x4 gv[NV], dv[NV];
     const float glv = a.gl[ri], dlv = a.dl[ri];
     float move = 0.0f;
-    if (!a.use_override) move = glv - a.glref[ri] - a.center[bank];
+    if (!a.use_override) {
+      // Every lane is here: r < R for all 128 rows of a query block or for none.
+      const int tiles = a.rows / kBlock;
+      const float centre = a.center != nullptr
+                               ? a.center[bank]
+                               : drift_centre(a.drift_part + (int64_t)bank * tiles, tiles, a.rows);
+      move = glv - a.glref[ri] - centre;
+    }
 #pragma unroll
     for (int i = 0; i < NV; ++i) gv[i] = *reinterpret_cast<const u32x4*>(gorow + col(i));
 #pragma unroll

@@ -454,52 +454,85 @@ hipError_t run_partial_reduce(const float* part, int banks, int groups, int elem
   return hipGetLastError();
 }
 
-// One workgroup per padded table row (bank, j), j < ntiles * 32: fold_rank of the rotated
-// variance (recap/sparse/closure.py:96-104), then w, kbar, vbar rounded to the query type
-// and written as row j of their tables, plain row-major D-element rows (rows j >= nb are
-// zero); the non-folded w row holds its columns in swap23 order.  FOLD writes w as the
-// kFoldCols-feature row [w_0 .. w_{r-1}, rho, rho, rho, 0 ...] (natural order), 32 bytes.
+// One launch for what lies between the closure statistics and the coarse tail, by block range:
+//   * C_vk (when cvk_part is given): the group partials summed in order, divided and rounded
+//     to the query type, 256 elements a block -- partial_reduce and basis_tables in one pass,
+//     with the same bits.  16 partials are requested at a time: the sum is a serial chain of
+//     `groups` loads otherwise (12.9 us for 86 groups).
+//   * the coarse tables, two padded table rows (bank, j), j < ntiles * 32, a block: fold_rank
+//     of the rotated variance (recap/sparse/closure.py:96-104), then w, kbar, vbar rounded to
+//     the query type and written as row j of their tables, plain row-major D-element rows
+//     (rows j >= nb are zero); the non-folded w row holds its columns in swap23 order.  FOLD
+//     writes w as the kFoldCols-feature row [w_0 .. w_{r-1}, rho, rho, rho, 0 ...] (natural
+//     order), 32 bytes.
+//   * one block that zeroes the attention launch's counters (when given).
 template <class T, int D, bool FOLD>
-__global__ __launch_bounds__(128) void tables_kernel(TablesArgs a) {
-  __shared__ float red[128];
-  __shared__ float vals[128];
+__global__ __launch_bounds__(256) void tables_kernel(TablesArgs a) {
+  __shared__ float red[256];
+  __shared__ float vals[256];
+  const int t = threadIdx.x;
+  const int cvk_blocks = a.cvk_part != nullptr ? a.banks * (D * D / 256) : 0;
+  int blk = blockIdx.x;
+  if (blk < cvk_blocks) {
+    const int64_t idx = (int64_t)blk * 256 + t;
+    const int64_t bank = idx / (D * D), e = idx % (D * D);
+    const float* p = a.cvk_part + bank * a.groups * (int64_t)(D * D) + e;
+    constexpr int kAhead = 16;
+    float acc = p[0];
+    for (int i0 = 1; i0 < a.groups; i0 += kAhead) {
+      float x[kAhead];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) x[i] = p[(int64_t)min(i0 + i, a.groups - 1) * (D * D)];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i)
+        if (i0 + i < a.groups) acc += x[i];
+    }
+    a.cvk_t[idx] = T::from_f(acc / a.divisor);
+    return;
+  }
+  blk -= cvk_blocks;
   const int ntiles = (a.nb + kCoarseSlots - 1) / kCoarseSlots;
-  const int bank = blockIdx.x / (ntiles * kCoarseSlots);
-  const int j = blockIdx.x % (ntiles * kCoarseSlots);
+  if (blk == a.banks * ntiles * (kCoarseSlots / 2)) {
+    for (int i = t; i < a.zero_words; i += 256) a.zero[i] = 0u;
+    return;
+  }
+  const int c = t & 127, half = t & 128;  // column, and the row's half of the scratch
+  const int rows = ntiles * kCoarseSlots, at_row = 2 * blk + (half >> 7);
+  const int bank = at_row / rows, j = at_row % rows;
   const bool real = j < a.nb;
   const int64_t row = (int64_t)bank * a.nb + j;
-  const int t = threadIdx.x;
-  const float v = (real && t < D) ? a.var[row * D + t] : 0.0f;
+  const float v = (real && c < D) ? a.var[row * D + c] : 0.0f;
   const bool fold = a.rank > 0 && a.rank < D;
-  red[t] = (fold && t >= a.rank && t < D) ? v : 0.0f;
+  red[t] = (fold && c >= a.rank && c < D) ? v : 0.0f;
   __syncthreads();
   for (int h = 64; h >= 1; h >>= 1) {
-    if (t < h) red[t] += red[t + h];
+    if (c < h) red[t] += red[t + h];
     __syncthreads();
   }
-  const float residual = fold ? red[0] / (float)(D - a.rank) : 0.0f;
-  vals[t] = (fold && t >= a.rank) ? residual : v;
+  const float residual = fold ? red[half] / (float)(D - a.rank) : 0.0f;
+  vals[t] = (fold && c >= a.rank) ? residual : v;
   __syncthreads();
-  if (t < D) {
-    // Row j of the bank's tables: element t of block j (zeros past the last block).
-    const int64_t at = ((int64_t)bank * ntiles * kCoarseSlots + j) * D + t;
-    a.kbar_t[at] = real ? T::from_f(a.kmean[row * D + t]) : (uint16_t)0;
-    a.vbar_t[at] = real ? T::from_f(a.vmean[row * D + t]) : (uint16_t)0;
+  if (c < D) {
+    // Row j of the bank's tables: element c of block j (zeros past the last block).
+    const int64_t at = (int64_t)at_row * D + c;
+    a.kbar_t[at] = real ? T::from_f(a.kmean[row * D + c]) : (uint16_t)0;
+    a.vbar_t[at] = real ? T::from_f(a.vmean[row * D + c]) : (uint16_t)0;
     if constexpr (FOLD) {
-      if (t < kFoldCols) {
-        const float f = t < a.rank ? vals[t] : (t < a.rank + 3 ? residual : 0.0f);
-        a.w_t[((int64_t)bank * ntiles * kCoarseSlots + j) * kFoldCols + t] =
-            real ? T::from_f(f) : (uint16_t)0;
+      if (c < kFoldCols) {
+        const float f = c < a.rank ? vals[t] : (c < a.rank + 3 ? residual : 0.0f);
+        a.w_t[(int64_t)at_row * kFoldCols + c] = real ? T::from_f(f) : (uint16_t)0;
       }
     } else {
-      a.w_t[at] = real ? T::from_f(vals[swap23(t)]) : (uint16_t)0;  // columns in swap23 order
+      a.w_t[at] = real ? T::from_f(vals[half + swap23(c)]) : (uint16_t)0;  // swap23 order
     }
   }
 }
 
 hipError_t run_tables(const TablesArgs& a, int dtype, hipStream_t s) {
   const int ntiles = (a.nb + kCoarseSlots - 1) / kCoarseSlots;
-  const dim3 grid((unsigned)(a.banks * ntiles * kCoarseSlots)), block(128);
+  const int cvk_blocks = a.cvk_part != nullptr ? a.banks * (a.dim * a.dim / 256) : 0;
+  const dim3 grid((unsigned)(cvk_blocks + a.banks * ntiles * (kCoarseSlots / 2) + (a.zero_words > 0 ? 1 : 0)));
+  const dim3 block(256);
   const bool fold = coarse_folded(dtype, a.dim, a.rank);
   if (dtype == BF16::code) {
     if (a.dim == 128) {

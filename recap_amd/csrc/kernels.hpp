@@ -48,6 +48,10 @@ hipError_t run_partial_reduce(const float* part, int banks, int groups, int elem
 struct TablesArgs {
   const float* var; const float* kmean; const float* vmean; int banks, nb, dim, rank;
   uint16_t* w_t; uint16_t* kbar_t; uint16_t* vbar_t;   // element type of the query
+  // Optional: C_vk in the query type from its partials [bank][groups][D][D], and counters to
+  // zero for a later launch of the same call.
+  const float* cvk_part; int groups; float divisor; uint16_t* cvk_t;
+  unsigned* zero; int zero_words;
 };
 
 // Folded w table of the coarse tail.  fold_rank leaves w with r + 1 distinct values per
@@ -106,6 +110,9 @@ struct AttnArgs {
   float* lse_native;                             // dense / dense-head [bank][N]
   int rows; const uint16_t* go; const float* gl; const uint16_t* det; const float* dl;
   const float* glref; const float* center; float alpha_override; int use_override;
+  // With center null: the coarse tail's partial sums of gl - glref, [bank][rows / 128], from
+  // which every wave takes its row's drift centre (the sum of drift_center).
+  const float* drift_part;
   unsigned* queue;   // kQueueWords zeroed words: per-XCD claim counters, or null (static)
   // Head and merge modes: segments of a long row (1: none), their states (attn_part_words(D)
   // 8-byte words each) and one zeroed arrival counter per long row.

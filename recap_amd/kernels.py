@@ -7,6 +7,8 @@ as raw device pointers with explicit strides.
 
 from __future__ import annotations
 
+import ctypes
+import functools
 import math
 from dataclasses import dataclass
 
@@ -367,11 +369,16 @@ def attn_split(banks: int, geo: Geometry, density: float = 0.25) -> int:
     return int(_lib.load().recap_attn_split(banks, geo.n_tokens, geo.n_video, float(density)))
 
 
+@functools.lru_cache(maxsize=256)
+def _attn_bytes(*sizes: int) -> int:
+    return int(_lib.load().recap_attn_workspace_size(*sizes))
+
+
 def _attn_workspace(q: torch.Tensor, geo: Geometry) -> tuple[int, torch.Tensor]:
     """(split, workspace) of a masked attention launch."""
     b, h, _, d = q.shape
     split = geo.attn_split or attn_split(b * h, geo)
-    size = int(_lib.load().recap_attn_workspace_size(b * h, d, geo.n_tokens, geo.n_video, split))
+    size = _attn_bytes(b * h, d, geo.n_tokens, geo.n_video, split)
     return split, torch.empty(size, dtype=torch.uint8, device=q.device)
 
 
@@ -439,6 +446,53 @@ def sparse_merge_attn(q: torch.Tensor, kv: PackedKV, rowmap: torch.Tensor,
          float(scale), _p(go), _p(gl), _p(det), _p(dl), _p(glref), _p(center), alpha,
          out.data_ptr(), out.stride(0), out.stride(1), out.stride(2), split, int(balance),
          work.data_ptr(), work.numel(), _stream())
+    return out
+
+
+@functools.lru_cache(maxsize=256)
+def _sparse_call_bytes(*sizes: int) -> int:
+    return int(_lib.load().recap_sparse_call_workspace_size(*sizes))
+
+
+def sparse_call(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rowmap: torch.Tensor,
+                geo: Geometry, scale: float, theta: float, rank: int, tables: BasisTables,
+                partition: torch.Tensor, kernel_mask: torch.Tensor, det: torch.Tensor,
+                dl: torch.Tensor, glref: torch.Tensor, alpha_override: float | None = None,
+                out: torch.Tensor | None = None, events=None) -> torch.Tensor:
+    """A whole corrected sparse call with a frozen basis in one library call and one
+    workspace: kv_pack, closure_stats, the tables, coarse_tail and sparse_merge_attn with
+    their outputs bit for bit, in five launches.  ``events``: five timing events recorded
+    before the first stage and after pack, closure (with the tables), coarse and attention."""
+    b, h, n, d = q.shape
+    banks = b * h
+    for name in ("u_hi_t", "u_lo_t", "u_t"):
+        table = getattr(tables, name)
+        if table.dtype != q.dtype:
+            raise ValueError(f"coarse_tail: table {name} is {table.dtype}, Q is {q.dtype}")
+        if table.numel() != banks * d * d:
+            raise ValueError(f"table {name} has {table.numel()} elements, expected {banks * d * d}")
+    partition, kernel_mask = partition.contiguous(), kernel_mask.contiguous()
+    if not (det.is_contiguous() and dl.is_contiguous() and glref.is_contiguous()):
+        raise ValueError("merge inputs must be contiguous")
+    if out is None:
+        out = torch.empty(b, h, n, d, dtype=q.dtype, device=q.device)
+    code = dtype_code(q.dtype)
+    group = geo.closure_group or closure_group(banks, geo.nb)
+    split = geo.attn_split or attn_split(banks, geo)
+    size = _sparse_call_bytes(code, banks, d, n, geo.n_video, group, rank, split)
+    work = torch.empty(size, dtype=torch.uint8, device=q.device)
+    handles = None
+    if events is not None:
+        for event in events:
+            event.record()   # creates the event; the call records it again at its stage
+        handles = (ctypes.c_void_p * 5)(*(event.cuda_event for event in events))
+    call("recap_sparse_call", q.data_ptr(), k.data_ptr(), v.data_ptr(), code, b, h, d,
+         *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], rowmap.data_ptr(), n, geo.n_video,
+         float(scale), float(theta), rank, group, tables.u_hi_t.data_ptr(),
+         tables.u_lo_t.data_ptr(), tables.u_t.data_ptr(), partition.data_ptr(),
+         kernel_mask.data_ptr(), det.data_ptr(), dl.data_ptr(), glref.data_ptr(),
+         -1.0 if alpha_override is None else float(alpha_override), out.data_ptr(),
+         *out.stride()[:3], split, handles, work.data_ptr(), size, _stream())
     return out
 
 

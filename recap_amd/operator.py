@@ -5,7 +5,8 @@
              minus coarse tail) and measures the error of the previous one.
 ``SPARSE``   the corrected sparse call: selected blocks exactly, the coarse tail over the
              omitted blocks, and the cached refinement weighted by the drift weight,
-             merged in log-mass space -- four HIP stages:
+             merged in log-mass space -- one library call (recap_sparse_call) of
+             four HIP stages:
 
     kv_pack          K/V gathered through the Hilbert row map into packed tiles + block means
     closure_stats    rotated block variances and C_vk (the frozen basis from the first call)
@@ -21,6 +22,7 @@ the reference's, so the diffusers processors call it unchanged.
 from __future__ import annotations
 
 import dataclasses
+import functools
 import math
 from dataclasses import dataclass, field
 
@@ -36,6 +38,7 @@ EXACT = "exact"
 REFRESH = "refresh"
 SPARSE = "sparse"
 _KINDS = (EXACT, REFRESH, SPARSE)
+_STAGES = ("start", "pack", "closure", "coarse", "attention")  # events of a timed SPARSE call
 
 
 class SparseAttention:
@@ -54,6 +57,16 @@ class SparseAttention:
     @property
     def basis(self) -> torch.Tensor | None:
         return self._basis
+
+    @property
+    def frozen(self) -> bool:
+        """The basis of the sample's first call is there."""
+        return self._basis is not None
+
+    @property
+    def tables(self) -> K.BasisTables | None:
+        """The frozen basis in the query type."""
+        return self._tables
 
     def head_partition(self, q: torch.Tensor, kv: K.PackedKV, rowmap: torch.Tensor,
                        geo: K.Geometry, scale: float) -> torch.Tensor:
@@ -190,6 +203,14 @@ def _publish_groups(bank: DetailBank, groups: list[DetailBank]) -> None:
         stats[0] if stats else None)
 
 
+@functools.lru_cache(maxsize=256)
+def _layer_geometry(n_tokens: int, n_video: int, banks: int, density: float) -> K.Geometry:
+    """A layer's block geometry with the choices that hold for every group of its heads."""
+    geo = K.Geometry(n_tokens=n_tokens, n_video=n_video)
+    return dataclasses.replace(geo, closure_group=K.closure_group(banks, geo.nb),
+                               attn_split=K.attn_split(banks, geo, density))
+
+
 @dataclass
 class Operator:
     """Dispatches one attention call per layer and owns the detail banks."""
@@ -273,12 +294,8 @@ class Operator:
 
     def _geometry(self, query: torch.Tensor) -> K.Geometry:
         self.layout._check(query)
-        banks = query.shape[0] * query.shape[1]
-        nb = -(-self.layout.video_tokens // K.BLOCK)
-        geo = K.Geometry(n_tokens=query.shape[-2], n_video=self.layout.video_tokens,
-                         closure_group=K.closure_group(banks, nb))
-        return dataclasses.replace(
-            geo, attn_split=K.attn_split(banks, geo, self.config.head_density))
+        return _layer_geometry(query.shape[-2], self.layout.video_tokens,
+                               query.shape[0] * query.shape[1], self.config.head_density)
 
     @torch.no_grad()
     def attend(self, layer_index: int, query: torch.Tensor, key: torch.Tensor,
@@ -455,37 +472,38 @@ class Operator:
 
     # -- sparse --------------------------------------------------------------------------
 
-    def _mark(self, name: str) -> None:
-        if self.stage_events is not None:
-            event = torch.cuda.Event(enable_timing=True)
-            event.record()
-            self.stage_events.setdefault(name, []).append(event)
-
     @torch.no_grad()
     def _sparse(self, layer, bank, q, k, v, geo, rowmap, out=None) -> torch.Tensor:
         """Head exactly, plus coarse tail and weighted cached refinement
-        (recap/operator.py:477-527), as four launches with the merge fused."""
+        (recap/operator.py:477-527), as one library call of five launches with the merge
+        fused."""
         if not bank.valid or bank.head_kernel_mask is None:
             raise RuntimeError("a sparse call was requested before an exact refresh")
         b, h, n, d = q.shape
         banks = b * h
         scale = K.scale_for(d)
-        self._mark("start")
+        if layer.frozen:
+            events = None
+            if self.stage_events is not None:
+                events = [torch.cuda.Event(enable_timing=True) for _ in _STAGES]
+                for name, event in zip(_STAGES, events):
+                    self.stage_events.setdefault(name, []).append(event)
+            return K.sparse_call(
+                q, k, v, rowmap, geo, scale, self.config.closure_gate_theta,
+                int(self.config.closure_rank), layer.tables,
+                bank.partition.reshape(banks, geo.nb, geo.nb), bank.head_kernel_mask, bank.value,
+                bank.log_mass, bank.coarse_lse, self.alpha_override, out, events)
+        # No basis yet (a bank that was handed in): stage by stage, the basis from these keys.
         kv = K.kv_pack(k, v, rowmap, geo)
-        self._mark("pack")
         context = layer.coarse_tail_context(kv, geo)
-        self._mark("closure")
         old_lse = bank.coarse_lse
         go, gl, drift_part = layer.coarse_tail_apply(
             q, rowmap, context, bank.partition.reshape(banks, geo.nb, geo.nb), geo, scale,
             glref=old_lse)
         center = K.drift_center(drift_part, geo) if geo.rows else None
-        self._mark("coarse")
-        out = K.sparse_merge_attn(q, kv, rowmap, bank.head_kernel_mask, geo, scale, go, gl,
-                                  bank.value, bank.log_mass, old_lse, center,
-                                  alpha_override=self.alpha_override, out=out)
-        self._mark("attention")
-        return out
+        return K.sparse_merge_attn(q, kv, rowmap, bank.head_kernel_mask, geo, scale, go, gl,
+                                   bank.value, bank.log_mass, old_lse, center,
+                                   alpha_override=self.alpha_override, out=out)
 
     # -- the refinement error ------------------------------------------------------------
 

@@ -581,3 +581,45 @@ def test_coarse_tail_extreme_partitions(cuda, name):
     assert not go.cpu()[erows].any()
     m, _ = metrics(gl.cpu()[fin], gl_ref[:, :rows][fin])
     assert m < 2e-3, m
+
+
+@pytest.mark.parametrize("name,dtype,rank,alpha", [
+    ("tiny", torch.bfloat16, 4, None),                  # folded w, whole blocks, no text
+    ("text-first-ragged", torch.float16, 4, None),      # full-width w, shared ragged block
+    ("text-last-d128", torch.bfloat16, 0, None),        # rank 0
+    ("text-last-d128", torch.bfloat16, 20, 0.5),        # full-width w, drift weight given
+    ("video-ragged-d128", torch.bfloat16, 4, None)])    # ragged, video only
+def test_sparse_call_equals_its_stages(cuda, name, dtype, rank, alpha):
+    """The one-call sparse path against the separate stage entry points on the same bank: the
+    same output bit for bit (its tables launch and the drift centre taken in the attention
+    waves included), for plain inputs and for transposed views of them."""
+    wl = SMALL[name]
+    print(f"case {name} {dtype} rank={rank} alpha={alpha}", flush=True)
+    q, k, v = make_qkv(wl, batch=2, seed=5, dtype=dtype, device=cuda)
+    layout = Layout.from_permutation(hilbert_permutation(wl.grid), text_tokens=wl.text_tokens,
+                                     text_first=wl.text_first)
+    rowmap, scale, theta = layout.rowmap(cuda), scale_for(wl.dim), 2.0
+    geo = K.Geometry(wl.tokens, wl.video_tokens, closure_group=2, attn_split=2)
+    kv = K.kv_pack(k, v, rowmap, geo)
+    part, kmask = K.pool_select(q, kv.k_means, rowmap, geo, wl.density, scale)
+    _, _, scatter = K.closure_stats(kv, geo, _lib.CLOSURE_CVK | _lib.CLOSURE_SCATTER)
+    tables = K.basis_tables(K.symmetric_eigen(scatter)[1], None, dtype, split=True, query=True)
+    g = torch.Generator().manual_seed(3)
+    banks = q.shape[0] * q.shape[1]
+    det = torch.randn(banks, geo.rows, wl.dim, generator=g).to(cuda, torch.float16)
+    dl = torch.randn(banks, geo.rows, generator=g).to(cuda)
+
+    var, cvk, _ = K.closure_stats(kv, geo, _lib.CLOSURE_ROT | _lib.CLOSURE_CVK, tables.u_hi_t,
+                                  tables.u_lo_t)
+    w, kbar, vbar = K.coarse_tables(var, kv, rank)
+    context = {"w": w, "kbar": kbar, "vbar": vbar, "u_t": tables.u_t, "rank": rank,
+               "cvk_t": K.basis_tables(None, cvk, dtype, cvk_table=True).cvk_t}
+    ref = torch.randn(banks, geo.rows, generator=g).to(cuda)
+    go, gl, drift = K.coarse_tail(q, rowmap, part, geo, context, scale, theta, ref)
+    want = K.sparse_merge_attn(q, kv, rowmap, kmask, geo, scale, go, gl, det, dl, ref,
+                               K.drift_center(drift, geo), alpha_override=alpha)
+    for views in (False, True):
+        x = [t.transpose(1, 2).contiguous().transpose(1, 2) if views else t for t in (q, k, v)]
+        got = K.sparse_call(*x, rowmap, geo, scale, theta, rank, tables, part, kmask, det, dl,
+                            ref, alpha)
+        assert torch.equal(got, want), views

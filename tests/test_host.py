@@ -132,6 +132,51 @@ def test_argument_validation_before_launch():
                   4097 * 128, 4097 * 128, 16, 0.125, 0.25, 16, 1 << 40, 16, 16, None)
 
 
+def test_sparse_call_is_checked_before_any_launch():
+    """recap_sparse_call rejects bad sizes, pointers, strides and workspaces on the host."""
+    lib = _lib.load()
+    size = lib.recap_sparse_call_workspace_size(_lib.RECAP_BF16, 2, 64, 512, 512, 1, 4, 1)
+    assert size > 0
+    for bad in [(9, 2, 64, 512, 512, 1, 4, 1), (_lib.RECAP_BF16, 0, 64, 512, 512, 1, 4, 1),
+                (_lib.RECAP_BF16, 2, 96, 512, 512, 1, 4, 1),
+                (_lib.RECAP_BF16, 2, 64, 500, 512, 1, 4, 1),
+                (_lib.RECAP_BF16, 2, 64, 512, 512, 0, 4, 1),
+                (_lib.RECAP_BF16, 2, 64, 512, 512, 1, 4, 9)]:
+        assert lib.recap_sparse_call_workspace_size(*bad) == -1
+    names = ["q", "k", "v", "dtype", "batch", "heads", "dim", "qb", "qh", "qn", "kb", "kh", "kn",
+             "vb", "vh", "vn", "rowmap", "n", "nv", "scale", "theta", "rank", "group", "uh", "ul",
+             "u", "part", "mask", "det", "dl", "ref", "alpha", "out", "ob", "oh", "on", "split",
+             "events", "work", "bytes", "stream"]
+    good = dict(zip(names, [16, 16, 16, _lib.RECAP_BF16, 1, 2, 64, 0, 0, 64, 0, 0, 64, 0, 0, 64,
+                            16, 512, 512, 0.125, 2.0, 4, 1, 16, 16, 16, 16, 16, 16, 16, 16, -1.0,
+                            16, 0, 0, 64, 1, None, 16, size, 0]))
+    for name, value in [("k", None), ("v", 8), ("kn", 3), ("out", None), ("rank", 65),
+                        ("rank", -1), ("group", 0), ("split", 9), ("theta", -1.0), ("scale", 0.0),
+                        ("u", None), ("uh", 8), ("part", None), ("mask", None), ("det", None),
+                        ("ref", None), ("work", None), ("work", 8), ("bytes", size - 1),
+                        ("n", 400), ("dim", 80), ("dtype", 7), ("rowmap", None)]:
+        with pytest.raises(ValueError):
+            _lib.call("recap_sparse_call", *{**good, name: value}.values())
+
+
+@pytest.mark.parametrize("banks,nt,nv,density", [(12, 4856, 4600, 0.2), (12, 32760, 32760, 0.4),
+                                                 (24, 119056, 118800, 0.2), (1, 262100, 261900, 0.1),
+                                                 (2, 4096, 4096, 0.25), (4, 1351, 1125, 0.25)])
+def test_attention_split_rule(banks, nt, nv, density):
+    """Segments of a long row: none without long rows or under 32 blocks, at most eight, none of
+    them under 16 blocks but for the last, and a workspace that grows with them."""
+    lib = _lib.load()
+    split = lib.recap_attn_split(banks, nt, nv, density)
+    tb, long_rows = -(-nt // 128), -(-nt // 128) - nv // 128
+    assert 1 <= split <= 8 and (split == 1 or long_rows > 0)
+    assert split == 1 or (tb + split - 1) / split >= 16 - 1
+    sizes = [lib.recap_attn_workspace_size(banks, 128, nt, nv, s) for s in range(1, 9)]
+    state = 128 * 128 * 4 + 256 * 8
+    assert all(b - a == banks * long_rows * state for a, b in zip(sizes[1:], sizes[2:]))
+    assert lib.recap_attn_split(banks, nt, nt + 1, density) == -1
+    assert lib.recap_attn_workspace_size(banks, 128, nt, nv, 9) == -1
+
+
 def test_workspace_queries():
     lib = _lib.load()
     assert lib.recap_closure_groups(118800, 8) == 117
