@@ -80,6 +80,22 @@ def test_indefinite_and_known_basis(cuda):
     _check(sym, lam, u)
 
 
+@pytest.mark.parametrize("n", [2, 3, 63, 64, 65, 128])
+def test_opposite_and_repeated_eigenvalues(cuda, n):
+    """Eigenvalues in exact pairs +s, -s, repeated ones, a rank-one matrix, a negative definite
+    one and the exchange matrix, at the edges of both kernels (64 and 128 in registers, other
+    orders in LDS), within the bounds above."""
+    g = torch.Generator().manual_seed(n)
+    q = torch.linalg.qr(torch.randn(4, n, n, generator=g, dtype=torch.float64))[0]
+    pairs = torch.arange(n, dtype=torch.float64) // 2 + 1
+    lv = torch.stack([pairs * (1 - 2 * (torch.arange(n) % 2)), pairs,
+                      torch.eye(n, dtype=torch.float64)[0] * 3, -pairs - 1])
+    a = ((q * lv.unsqueeze(-2)) @ q.transpose(-1, -2)).float()
+    a = torch.cat([a, torch.eye(n).flip(0).expand(1, n, n)])
+    lam, u = K.symmetric_eigen(a.to(cuda))
+    _check(a, lam, u)
+
+
 def test_diagonal_zero_and_identity(cuda):
     n = 64
     diag = torch.diag_embed(torch.tensor([[float((7 * i) % n) for i in range(n)]]))
