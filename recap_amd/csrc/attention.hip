@@ -456,7 +456,10 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
       }
     }
   }
-  const int nsub = MODE == kModeDenseHead ? 2 * a.tb : 2 * nkeep;  // 64-key sub-tiles
+  int nsub = MODE == kModeDenseHead ? 2 * a.tb : 2 * nkeep;  // 64-key sub-tiles
+  // Opaque: told that nsub is 2 nkeep, the compiler rewrites the d = 64 walk's loop over both
+  // and spills 90 registers in it.
+  asm volatile("" : "+s"(nsub));
 
   // Sub-tile `it` = half (it & 1) of kept tile (it >> 1): its K rows and its V^T half are
   // each HALF contiguous bytes of the packed images, copied verbatim into LDS slot it & 1
@@ -481,7 +484,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
 
   if (nsub > 0) {
     copy(krs, image(0), k_lds0);
-    copy(vrs, image(0), v_lds0);
+    if constexpr (D != 64) copy(vrs, image(0), v_lds0);   // (at d = 64 its step copies it)
   }
   if (nsub > 1) copy(krs, image(1), k_lds1);
   tile_barrier();
@@ -513,14 +516,15 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
   };
   // Keys past the sequence end in a sub-tile of the last (ragged) block.
   auto mask_tail = [&](f32x16 (&s)[kGroups][2], int it) {
-    const int limit = a.n_tokens - ((a.tb - 1) * kBlock + 64 * (it & 1));
+    int limit = a.n_tokens - ((a.tb - 1) * kBlock + 64 * (it & 1)) - 4 * g;
+    asm volatile("" : "+v"(limit));  // keeps the compares in this rare branch
 #pragma unroll
     for (int q = 0; q < kGroups; ++q)
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int rr = 0; rr < 16; ++rr)
-          if (32 * kt + mfma_row(rr, g) >= limit) s[q][kt][rr] = -INFINITY;
+          if (32 * kt + mfma_row(rr, 0) >= limit) s[q][kt][rr] = -INFINITY;
   };
   // Lazy running-max update of group q from a per-lane candidate raw score: moves only when
   // the row max grows by more than kRescaleSlack, rescaling O and l.  The test is on raw
@@ -577,7 +581,6 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
                   auto next_tag, auto parity_tag) __attribute__((always_inline)) {
     constexpr bool kNext = decltype(next_tag)::value;
     constexpr bool kOdd = decltype(parity_tag)::value;
-    constexpr bool kSumCheck = D == 64;
     if (it + 1 < nsub) copy(vrs, image(it + 1), kOdd ? v_lds0 : v_lds1);
     if (it + 2 < nsub) copy(krs, image(it + 2), kOdd ? k_lds1 : k_lds0);
     const char* kl = kOdd ? k_lds0 : k_lds1;   // K_{it+1}
@@ -616,43 +619,6 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
           part[q][kt] = (pp & 7) ? part[q][kt] + (p0 + p1) : p0 + p1;
           w[q][kt][hh][e >> 1] = pack2<T>(p0, p1);
         }
-        if constexpr (kSumCheck) {
-          // After the slice with the last pair, before any PV MFMA reads them: a lane whose
-          // probabilities overflow the cap (or are not finite, as when m = -inf) redoes the
-          // sub-tile against the raised running max, rescaling O and l first.
-          if ((n + 1) * PPS >= NPAIR) {
-            bool over = false;
-#pragma unroll
-            for (int q = 0; q < kGroups; ++q) over |= !(part[q][0] + part[q][1] <= kSumCap);
-            if (__any(over)) {
-              __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-              for (int q = 0; q < kGroups; ++q) {
-                float mx = -INFINITY;
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                  for (int rr = 0; rr < 16; ++rr) mx = __builtin_elementwise_maximum(mx, cur[q][kt][rr]);
-                const float mnew = pair_max(mx) * a.scale_log2;
-                if (mnew > m[q]) {
-                  const float alpha = __builtin_amdgcn_exp2f(m[q] - mnew);
-                  lsum[q] *= alpha;
-#pragma unroll
-                  for (int dt = 0; dt < NDT; ++dt) oacc[q][dt] *= alpha;
-                  m[q] = mnew;
-                }
-#pragma unroll
-                for (int pp = 0; pp < 16; ++pp) {
-                  const int kt = pp >> 3, hh = (pp >> 2) & 1, e = 2 * (pp & 3);
-                  const float p0 = __builtin_amdgcn_exp2f(fmaf(cur[q][kt][8 * hh + e], a.scale_log2, -m[q]));
-                  const float p1 = __builtin_amdgcn_exp2f(fmaf(cur[q][kt][8 * hh + e + 1], a.scale_log2, -m[q]));
-                  part[q][kt] = (pp & 7) ? part[q][kt] + (p0 + p1) : p0 + p1;
-                  w[q][kt][hh][e >> 1] = pack2<T>(p0, p1);
-                }
-              }
-            }
-          }
-        }
       }
       if (n < NQK) {
         const int st = n >> 1, kt = n & 1;
@@ -672,7 +638,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
           const u32x4 pk = {w[q][kt][hh][0], w[q][kt][hh][1], w[q][kt][hh][2], w[q][kt][hh][3]};
           oacc[q][dt] = T::mfma32(fr[n % 3], pk, oacc[q][dt]);
         }
-        if constexpr (kNext && !kSumCheck) {
+        if constexpr (kNext) {
           // Row max over MPS pairs of S_{it+1} scores (pair mp: group mp % kGroups).
 #pragma unroll
           for (int mp = i * MPS; mp < (i + 1) * MPS; ++mp) {
@@ -688,7 +654,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
     if constexpr (MODE == kModeDenseHead) {
       if (it + 1 == kept_end) store_head();
     }
-    if constexpr (kNext && !kSumCheck) {
+    if constexpr (kNext) {
 #pragma unroll
       for (int q = 0; q < kGroups; ++q) update_max(q, mx[q]);
     }
@@ -700,6 +666,98 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
     const int j = MODE == kModeDense ? (it >> 1) : __builtin_amdgcn_readfirstlane(list[first + (it >> 1)]);
     return ragged && j == a.tb - 1;
   };
+  // The d = 64 step.  Its softmax work exceeds its matrix work, so the two are pipelined one
+  // sub-tile further apart than above: step `it` computes P_it on the VALU while the matrix core
+  // runs S_{it+1} and PV_{it-1}, which do not depend on it, alternately.  Slice n issues one
+  // MFMA (with the LDS fragment read four slices before) and its share of the P pairs.  The
+  // running max is checked and raised at the end of the step, when O holds the sub-tiles before
+  // `it`.  (With P and PV of one sub-tile in one step, as above, the PV half of a step had no
+  // VALU work and waited for each fragment.  A refresh at 48 heads x 24,706 tokens 19.66 -> 19.38
+  // ms, a sparse call at 2 x 4,096 47.8 -> 46.4 us, and no change at 48 x 45,106, where power
+  // bounds both forms; the same bits.)
+  // `vt` and `kt_next` are the key tiles of sub-tiles it and it + 2.
+  auto step64 = [&](int it, int vt, int kt_next, f32x16 (&cur)[kGroups][2],
+                    f32x16 (&nxt)[kGroups][2], u32x4 (&w)[4], u32x4 (&wp)[4],
+                    bool mask, auto next_tag, auto pv_tag, auto parity_tag) __attribute__((always_inline)) {
+    static_assert(kGroups == 1, "one query group per wave");
+    constexpr bool kNext = decltype(next_tag)::value;
+    constexpr bool kPV = decltype(pv_tag)::value;
+    constexpr bool kOdd = decltype(parity_tag)::value;
+    constexpr int half = kOdd ? HALF : 0;
+    copy(vrs, vt * G::kTileBytes + half, kOdd ? v_lds1 : v_lds0);   // V_it, read in the next step
+    if (it + 2 < nsub) copy(krs, kt_next * G::kTileBytes + half, kOdd ? k_lds1 : k_lds0);
+    const char* kl = kOdd ? k_lds0 : k_lds1;   // K_{it+1}
+    const char* vl = kOdd ? v_lds0 : v_lds1;   // V_{it-1}
+    constexpr int NQK = 2 * NS, NPV = 4 * NDT;
+    constexpr int NN = (kNext ? NQK : 0) + (kPV ? NPV : 0);
+    // MFMA n: alternately S and PV where there are both.
+    auto is_qk = [](int n) { return kNext && (!kPV || n % 2 == 0); };
+    auto frag = [&](int n) -> u32x4 {
+      const int i = kNext && kPV ? n / 2 : n;
+      if (is_qk(n)) return lds_load16(kl, G::k_off(32 * (i & 1) + l32, 2 * (i >> 1) + g));
+      return lds_load16(vl, G::vt_off(32 * (i % NDT) + l32, 2 * (i / NDT) + g));
+    };
+    constexpr int kAhead = 4;
+    u32x4 fr[kAhead + 1];
+#pragma unroll
+    for (int n = 0; n < kAhead; ++n) fr[n] = frag(n);
+    float part[2];
+    auto pair = [&](int pp) {
+      const int kt = pp >> 3, hh = (pp >> 2) & 1, e = 2 * (pp & 3);
+      const float p0 = __builtin_amdgcn_exp2f(fmaf(cur[0][kt][8 * hh + e], a.scale_log2, -m[0]));
+      const float p1 = __builtin_amdgcn_exp2f(fmaf(cur[0][kt][8 * hh + e + 1], a.scale_log2, -m[0]));
+      part[kt] = (pp & 7) ? part[kt] + (p0 + p1) : p0 + p1;
+      w[2 * kt + hh][e >> 1] = pack2<T>(p0, p1);
+    };
+    constexpr int PPS = 16 / NN;  // P pairs per slice
+#pragma unroll
+    for (int n = 0; n < NN; ++n) {
+      if (n + kAhead < NN) fr[(n + kAhead) % (kAhead + 1)] = frag(n + kAhead);
+      const u32x4 f = fr[n % (kAhead + 1)];
+      const int i = kNext && kPV ? n / 2 : n;
+      if (is_qk(n)) {
+        const int st = i >> 1, kt = i & 1;
+        nxt[0][kt] = T::mfma32(f, qreg[0][st], st == 0 ? f32x16{} : nxt[0][kt]);
+      } else {
+        oacc[0][i % NDT] = T::mfma32(f, wp[i / NDT], oacc[0][i % NDT]);
+      }
+#pragma unroll
+      for (int pp = n * PPS; pp < (n + 1) * PPS; ++pp) {
+        pair(pp);
+        // Packed and summed here, not after the branches below (which would keep every P alive).
+        if ((pp & 3) == 3) asm volatile("" : "+v"(w[pp >> 2]), "+v"(part[pp >> 3]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (mask) {  // S_{it+1} in the ragged last block (a rare uniform branch)
+      mask_tail(nxt, it + 1);
+    }
+    if constexpr (MODE == kModeDenseHead) {
+      if (it == kept_end) store_head();
+    }
+    // A lane whose probabilities overflow the cap (or are not finite, as when m = -inf) redoes
+    // the sub-tile against the raised running max, rescaling O and l first.
+    if (__any(!(part[0] + part[1] <= kSumCap))) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr) mx = __builtin_elementwise_maximum(mx, cur[0][kt][rr]);
+      const float mnew = pair_max(mx) * a.scale_log2;
+      if (mnew > m[0]) {
+        const float alpha = __builtin_amdgcn_exp2f(m[0] - mnew);
+        lsum[0] *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) oacc[0][dt] *= alpha;
+        m[0] = mnew;
+      }
+#pragma unroll
+      for (int pp = 0; pp < 16; ++pp) pair(pp);
+    }
+    lsum[0] += part[0] + part[1];
+    tile_barrier();
+  };
+
   f32x16 sa[kGroups][2], sb[kGroups][2];
   if (nsub > 0) {
     qk(k_lds0, sa);
@@ -709,13 +767,44 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
   }
   using F = std::false_type;
   using Tr = std::true_type;
+  if (MODE == kModeDenseHead && kept_end == 0) store_head();
+  if constexpr (D == 64) {
+    // Steps 0 .. nsub - 1 (nsub is even) and PV of the last sub-tile.  Steps 2 i and 2 i + 1 copy
+    // V of walk tile i and K of tile i + 1; each list entry is read a pair of steps early.  A
+    // ragged block's sub-tiles are the first two (kept, in the masked modes) or the last two.
+    if (nsub >= 2) {
+      const int ntile = nsub >> 1;
+      auto tile = [&](int i) {
+        const int j = min(i, ntile - 1);
+        return MODE == kModeDense ? j : __builtin_amdgcn_readfirstlane(list[first + j]);
+      };
+      u32x4 wa[4], wb[4];
+      int j0 = tile(0), j1 = tile(1);
+      const bool tail = nsub >= 4 && ragged_at(nsub - 1);
+      step64(0, j0, j1, sa, sb, wa, wb, ragged_at(1), Tr{}, F{}, F{});
+      for (int it = 1; it + 2 < nsub; it += 2) {
+        const int j2 = tile((it + 3) >> 1);
+        const bool mask = tail && it + 3 == nsub;
+        step64(it, j0, j1, sb, sa, wb, wa, mask, Tr{}, Tr{}, Tr{});
+        step64(it + 1, j1, j2, sa, sb, wa, wb, mask, Tr{}, Tr{}, F{});
+        j0 = j1;
+        j1 = j2;
+      }
+      step64(nsub - 1, j0, j1, sb, sa, wb, wa, false, F{}, Tr{}, Tr{});
+#pragma unroll
+      for (int i = 0; i < 4 * NDT; ++i) {
+        const u32x4 f = lds_load16(v_lds1, G::vt_off(32 * (i % NDT) + l32, 2 * (i / NDT) + g));
+        oacc[0][i % NDT] = T::mfma32(f, wb[i / NDT], oacc[0][i % NDT]);
+      }
+      if (MODE == kModeDenseHead && kept_end == nsub) store_head();
+    }
+  } else {
   // Steps go in pairs (even step: S in sa -> sb, odd step: sb -> sa) so each array keeps one
   // role.  Step it computes S of sub-tile it + 1, masked when that sub-tile lies in the ragged
   // last block: in the masked modes a kept ragged block goes first (sub-tiles 0 and 1), and in
   // dense mode, or in dense-head mode when the mask drops it, the ragged block goes last, so
   // only the first and the last two pairs are peeled and the main loop runs unmasked.  The
   // final step has no next sub-tile.
-  if (MODE == kModeDenseHead && kept_end == 0) store_head();
   int it = 0;
   if constexpr (MODE != kModeDense) {
     if (nsub >= 4) {
@@ -736,6 +825,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
   if (nsub >= 2) {
     step(it, sa, sb, ragged_at(it + 1), Tr{}, F{});
     step(it + 1, sb, sa, false, F{}, Tr{});
+  }
   }
 
   constexpr int kStore = MODE == kModeDenseHead ? kModeDense : MODE;
