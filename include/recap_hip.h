@@ -281,9 +281,27 @@ int recap_sparse_merge_attn_ws(const void* q, int dtype, int64_t batch, int64_t 
                                int64_t out_stride_n, int64_t split, int balance,
                                void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The per-call closure statistics and the tables of the coarse tail in two launches: the
+ * rotated variances (ROT) and C_vk (CVK) of recap_closure_stats, C_vk summed, divided by
+ * n_video and rounded to `dtype` (cvk_t [banks, dim, dim]), and the tables of
+ * recap_coarse_tables.  A partial of C_vk covers `group` blocks, accumulated as `parts` runs
+ * whose sums are added in order; a call with few heads computes one partial per run instead
+ * (recap_closure_partials(..) of [dim, dim] in all), with the same bits, so the heads of a
+ * layer may be called in groups.  recap_closure_span gives group and parts for a layer of
+ * `banks` heads.
+ * Replaces recap/sparse/attention.py:154-202 for a frozen basis. */
+int recap_closure_span(int64_t banks, int64_t n_video, int64_t* group, int64_t* parts);
+int64_t recap_closure_partials(int64_t banks, int64_t n_video, int64_t group, int64_t parts);
+int recap_closure_tables(const void* k_tiles, const void* vt_tiles, const float* k_means,
+                         const float* v_means, int dtype, const void* u_hi_t, const void* u_lo_t,
+                         int64_t banks, int64_t dim, int64_t n_tokens, int64_t n_video,
+                         int64_t group, int64_t parts, int64_t rank, float* variance,
+                         float* cvk_partial, void* cvk_t, void* w, void* kbar, void* vbar,
+                         void* stream);
+
 /* A whole corrected sparse call of a layer with a frozen basis, as five launches on `stream`:
- * recap_kv_pack, recap_closure_stats (ROT | CVK, `group` blocks a workgroup), the C_vk and
- * coarse tables in one launch that also zeroes the attention counters, recap_coarse_tail and
+ * recap_kv_pack, the two of recap_closure_tables (the second also zeroes the attention
+ * counters), recap_coarse_tail and
  * recap_sparse_merge_attn_ws, whose waves take the drift centre from the coarse tail's partial
  * sums.  Outputs are those of the separate calls, bit for bit.  `u_hi_t`, `u_lo_t` and `u_t`
  * are the tables of recap_basis_tables; `det`, `dl`, `glref`, `partition` and `kernel_mask`
@@ -293,15 +311,15 @@ int recap_sparse_merge_attn_ws(const void* q, int dtype, int64_t batch, int64_t 
  * Nothing is launched when an argument is rejected.
  * Replaces Operator._sparse, recap/operator.py:477-527. */
 int64_t recap_sparse_call_workspace_size(int dtype, int64_t banks, int64_t dim, int64_t n_tokens,
-                                         int64_t n_video, int64_t group, int64_t rank,
-                                         int64_t split);
+                                         int64_t n_video, int64_t group, int64_t parts,
+                                         int64_t rank, int64_t split);
 int recap_sparse_call(const void* q, const void* k, const void* v, int dtype, int64_t batch,
                       int64_t heads, int64_t dim, int64_t q_stride_b, int64_t q_stride_h,
                       int64_t q_stride_n, int64_t k_stride_b, int64_t k_stride_h,
                       int64_t k_stride_n, int64_t v_stride_b, int64_t v_stride_h,
                       int64_t v_stride_n, const int32_t* rowmap, int64_t n_tokens,
                       int64_t n_video, float scale, float theta, int64_t rank, int64_t group,
-                      const void* u_hi_t, const void* u_lo_t, const void* u_t,
+                      int64_t parts, const void* u_hi_t, const void* u_lo_t, const void* u_t,
                       const uint8_t* partition, const uint8_t* kernel_mask, const void* det,
                       const float* dl, const float* glref, float alpha_override, void* out,
                       int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_n,

@@ -57,10 +57,15 @@ SIGNATURES: dict[str, tuple] = {
     "recap_sparse_merge_attn": (_I, [_P, _I, _I64, _I64, _I64, *_STRIDES, _P, _P, _P, _P, _I64,
                                      _I64, _F, _P, _P, _P, _P, _P, _P, _F, _P, *_STRIDES, _P, _P]),
     "recap_attn_queue_words": (_I64, []),
-    "recap_sparse_call_workspace_size": (_I64, [_I, _I64, _I64, _I64, _I64, _I64, _I64, _I64]),
+    "recap_closure_span": (_I, [_I64, _I64, _P, _P]),
+    "recap_closure_partials": (_I64, [_I64, _I64, _I64, _I64]),
+    "recap_closure_tables": (_I, [_P, _P, _P, _P, _I, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64,
+                                  _I64, _P, _P, _P, _P, _P, _P, _P]),
+    "recap_sparse_call_workspace_size": (_I64, [_I, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
+                                                _I64]),
     "recap_sparse_call": (_I, [_P, _P, _P, _I, _I64, _I64, _I64, *_STRIDES, *_STRIDES, *_STRIDES,
-                               _P, _I64, _I64, _F, _F, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P,
-                               _F, _P, *_STRIDES, _I64, _P, _P, _I64, _P]),
+                               _P, _I64, _I64, _F, _F, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P,
+                               _P, _P, _F, _P, *_STRIDES, _I64, _P, _P, _I64, _P]),
     "recap_attn_split": (_I64, [_I64, _I64, _I64, ctypes.c_double]),
     "recap_attn_workspace_size": (_I64, [_I64, _I64, _I64, _I64, _I64]),
     "recap_block_sparse_attn_ws": (_I, [_P, _I, _I64, _I64, _I64, *_STRIDES, _P, _P, _P, _P,

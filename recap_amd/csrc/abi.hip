@@ -632,18 +632,88 @@ int recap_sparse_merge_attn_ws(const void* q, int dtype, int64_t batch, int64_t 
   return hip_status(run_attention(a, dtype, (int)dim, kModeMerge, as_stream(stream)), "attention launch");
 }
 
+static int64_t cvk_partials(int64_t banks, int64_t nb, ClosureSpan span) {
+  const int64_t groups = (nb + span.group - 1) / span.group;
+  return banks * groups * (closure_fine(banks, nb, span) ? span.parts : 1);
+}
+
+// The closure statistics and the tables of the coarse tail, two launches; arguments checked.
+static int closure_and_tables(const void* k_tiles, const void* vt_tiles, const float* k_means,
+                              const float* v_means, int dtype, const void* u_hi_t,
+                              const void* u_lo_t, int64_t banks, int64_t dim, const Geom& g,
+                              int64_t n_video, ClosureSpan span, int64_t rank, float* variance,
+                              float* cvk_partial, void* cvk_t, void* w, void* kbar, void* vbar,
+                              unsigned* zero, int zero_words, hipStream_t s) {
+  ClosureArgs a{};
+  a.kp = static_cast<const uint16_t*>(k_tiles); a.vp = static_cast<const uint16_t*>(vt_tiles);
+  a.kmean = k_means;
+  a.u_hi_t = static_cast<const uint16_t*>(u_hi_t); a.u_lo_t = static_cast<const uint16_t*>(u_lo_t);
+  a.banks = (int)banks; a.nb = (int)g.nb; a.tb = (int)g.tb; a.n_video = (int)n_video;
+  a.group = span.group; a.groups = (int)((g.nb + span.group - 1) / span.group);
+  a.parts = span.parts; a.fine = closure_fine(banks, g.nb, span) ? 1 : 0;
+  a.var = variance; a.cvk_part = cvk_partial;
+  CHECK(hip_status(run_closure(a, dtype, (int)dim, kRot | kCvk, s), "closure launch"));
+  TablesArgs t{};
+  t.var = variance; t.kmean = k_means; t.vmean = v_means;
+  t.banks = (int)banks; t.nb = (int)g.nb; t.dim = (int)dim; t.rank = (int)rank;
+  t.w_t = static_cast<uint16_t*>(w); t.kbar_t = static_cast<uint16_t*>(kbar);
+  t.vbar_t = static_cast<uint16_t*>(vbar);
+  t.cvk_part = cvk_partial; t.groups = a.groups; t.runs = a.fine ? span.parts : 1;
+  t.divisor = (float)n_video; t.cvk_t = static_cast<uint16_t*>(cvk_t);
+  t.zero = zero; t.zero_words = zero_words;
+  return hip_status(run_tables(t, dtype, s), "tables launch");
+}
+
+static int check_span(int64_t group, int64_t parts) {
+  REQUIRE(group >= 1 && group <= 4096 && parts >= 1 && parts <= 64, "bad closure group %lld / parts %lld",
+          (long long)group, (long long)parts);
+  return RECAP_OK;
+}
+
+int recap_closure_span(int64_t banks, int64_t n_video, int64_t* group, int64_t* parts) {
+  REQUIRE(banks >= 1 && n_video >= 1 && group && parts, "bad banks/n_video or NULL output");
+  const ClosureSpan span = closure_span(banks, (n_video + kBlock - 1) / kBlock);
+  *group = span.group;
+  *parts = span.parts;
+  return RECAP_OK;
+}
+
+int64_t recap_closure_partials(int64_t banks, int64_t n_video, int64_t group, int64_t parts) {
+  if (banks < 1 || n_video < 1 || check_span(group, parts) != RECAP_OK) return -1;
+  return cvk_partials(banks, (n_video + kBlock - 1) / kBlock, {(int)group, (int)parts});
+}
+
+int recap_closure_tables(const void* k_tiles, const void* vt_tiles, const float* k_means,
+                         const float* v_means, int dtype, const void* u_hi_t, const void* u_lo_t,
+                         int64_t banks, int64_t dim, int64_t n_tokens, int64_t n_video,
+                         int64_t group, int64_t parts, int64_t rank, float* variance,
+                         float* cvk_partial, void* cvk_t, void* w, void* kbar, void* vbar,
+                         void* stream) {
+  CHECK(check_common(dtype, dim));
+  CHECK(check_tokens(n_tokens, n_video));
+  REQUIRE(banks >= 1 && rank >= 0, "bad banks/rank");
+  CHECK(check_span(group, parts));
+  REQUIRE(k_tiles && vt_tiles && aligned16(k_tiles) && aligned16(vt_tiles) && k_means && v_means,
+          "tiles/means");
+  REQUIRE(u_hi_t && u_lo_t && aligned16(u_hi_t) && aligned16(u_lo_t), "u_hi_t, u_lo_t");
+  REQUIRE(variance && cvk_partial && cvk_t && w && kbar && vbar, "NULL output");
+  return closure_and_tables(k_tiles, vt_tiles, k_means, v_means, dtype, u_hi_t, u_lo_t, banks, dim,
+                            geometry(n_tokens, n_video), n_video, {(int)group, (int)parts}, rank,
+                            variance, cvk_partial, cvk_t, w, kbar, vbar, nullptr, 0,
+                            as_stream(stream));
+}
+
 // Workspace of recap_sparse_call: byte offsets of its parts.
 struct SparseSpace {
   int64_t kt, vt, km, vm, var, cvk_t, w, kbar, vbar, cvk_part, go, gl, drift, attn, attn_bytes, bytes;
 };
 
 static SparseSpace sparse_space(int dtype, int64_t banks, int64_t dim, const Geom& g, int64_t n_video,
-                                int64_t group, int64_t rank, int64_t split) {
+                                ClosureSpan span, int64_t rank, int64_t split) {
   SparseSpace w;
   int64_t at = 0;
   auto take = [&](int64_t bytes) { const int64_t o = at; at += align256(bytes); return o; };
   const int64_t padded = (g.nb + kCoarseSlots - 1) / kCoarseSlots * kCoarseSlots;
-  const int64_t groups = (g.nb + group - 1) / group;
   w.kt = take(banks * g.tb * kBlock * dim * 2);
   w.vt = take(banks * g.tb * kBlock * dim * 2);
   w.km = take(banks * g.nb * dim * 4);
@@ -654,7 +724,7 @@ static SparseSpace sparse_space(int dtype, int64_t banks, int64_t dim, const Geo
   w.kbar = take(banks * padded * dim * 2);
   w.vbar = take(banks * padded * dim * 2);
   // The C_vk partials are read before the coarse output is written.
-  w.cvk_part = w.go = take(std::max(banks * groups * dim * dim * 4, banks * g.rows * dim * 2));
+  w.cvk_part = w.go = take(std::max(cvk_partials(banks, g.nb, span) * dim * dim * 4, banks * g.rows * dim * 2));
   w.gl = take(banks * g.rows * 4);
   w.drift = take(banks * (g.rows / kBlock) * 4);
   w.attn_bytes = attn_space(banks, dim, g.tb - first_long(g, n_video), split).bytes;
@@ -664,12 +734,13 @@ static SparseSpace sparse_space(int dtype, int64_t banks, int64_t dim, const Geo
 }
 
 int64_t recap_sparse_call_workspace_size(int dtype, int64_t banks, int64_t dim, int64_t n_tokens,
-                                         int64_t n_video, int64_t group, int64_t rank,
-                                         int64_t split) {
+                                         int64_t n_video, int64_t group, int64_t parts,
+                                         int64_t rank, int64_t split) {
   if (check_common(dtype, dim) != RECAP_OK || check_tokens(n_tokens, n_video) != RECAP_OK ||
-      banks < 1 || group < 1 || rank < 0 || split < 1 || split > kMaxSplit)
+      banks < 1 || check_span(group, parts) != RECAP_OK || rank < 0 || split < 1 || split > kMaxSplit)
     return -1;
-  return sparse_space(dtype, banks, dim, geometry(n_tokens, n_video), n_video, group, rank, split).bytes;
+  return sparse_space(dtype, banks, dim, geometry(n_tokens, n_video), n_video,
+                      {(int)group, (int)parts}, rank, split).bytes;
 }
 
 int recap_sparse_call(const void* q, const void* k, const void* v, int dtype, int64_t batch,
@@ -678,7 +749,7 @@ int recap_sparse_call(const void* q, const void* k, const void* v, int dtype, in
                       int64_t k_stride_n, int64_t v_stride_b, int64_t v_stride_h,
                       int64_t v_stride_n, const int32_t* rowmap, int64_t n_tokens,
                       int64_t n_video, float scale, float theta, int64_t rank, int64_t group,
-                      const void* u_hi_t, const void* u_lo_t, const void* u_t,
+                      int64_t parts, const void* u_hi_t, const void* u_lo_t, const void* u_t,
                       const uint8_t* partition, const uint8_t* kernel_mask, const void* det,
                       const float* dl, const float* glref, float alpha_override, void* out,
                       int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_n,
@@ -693,14 +764,15 @@ int recap_sparse_call(const void* q, const void* k, const void* v, int dtype, in
   REQUIRE(aligned16(u_hi_t) && aligned16(u_lo_t) && aligned16(u_t), "tables must be 16-byte aligned");
   REQUIRE(theta >= 0.0f, "theta must be non-negative");
   REQUIRE(rank >= 0 && rank <= dim, "rank %lld outside [0, dim]", (long long)rank);
-  REQUIRE(group >= 1, "bad group");
+  CHECK(check_span(group, parts));
+  const ClosureSpan span = {(int)group, (int)parts};
   REQUIRE(split >= 1 && split <= kMaxSplit, "split %lld outside 1..%d", (long long)split, kMaxSplit);
   REQUIRE(workspace != nullptr && aligned16(workspace), "workspace must be non-NULL and 16-byte aligned");
   const Geom g = geometry(n_tokens, n_video);
   REQUIRE(g.nb <= 4096, "too many video blocks (%lld > 4096)", (long long)g.nb);
   REQUIRE(batch >= 1 && heads >= 1, "bad batch/heads");
   const int64_t banks = batch * heads;
-  const SparseSpace w = sparse_space(dtype, banks, dim, g, n_video, group, rank, split);
+  const SparseSpace w = sparse_space(dtype, banks, dim, g, n_video, span, rank, split);
   REQUIRE(workspace_bytes >= w.bytes, "workspace of %lld bytes, need %lld",
           (long long)workspace_bytes, (long long)w.bytes);
   char* base = static_cast<char*>(workspace);
@@ -728,19 +800,10 @@ int recap_sparse_call(const void* q, const void* k, const void* v, int dtype, in
                       v_stride_b, v_stride_h, v_stride_n, rowmap, n_tokens, n_video, base + w.kt,
                       base + w.vt, f32(w.km), f32(w.vm), stream));
   CHECK(mark(1));
-  CHECK(recap_closure_stats(base + w.kt, base + w.vt, f32(w.km), dtype, u_hi_t, u_lo_t, banks, dim,
-                            n_tokens, n_video, group, RECAP_CLOSURE_ROT | RECAP_CLOSURE_CVK,
-                            f32(w.var), f32(w.cvk_part), nullptr, stream));
-  TablesArgs t{};
-  t.var = f32(w.var); t.kmean = f32(w.km); t.vmean = f32(w.vm);
-  t.banks = (int)banks; t.nb = (int)g.nb; t.dim = (int)dim; t.rank = (int)rank;
-  t.w_t = reinterpret_cast<uint16_t*>(base + w.w);
-  t.kbar_t = reinterpret_cast<uint16_t*>(base + w.kbar);
-  t.vbar_t = reinterpret_cast<uint16_t*>(base + w.vbar);
-  t.cvk_part = f32(w.cvk_part); t.groups = (int)recap_closure_groups(n_video, group);
-  t.divisor = (float)n_video; t.cvk_t = reinterpret_cast<uint16_t*>(base + w.cvk_t);
-  t.zero = words; t.zero_words = (int)space.counters;
-  CHECK(hip_status(run_tables(t, dtype, s), "tables launch"));
+  CHECK(closure_and_tables(base + w.kt, base + w.vt, f32(w.km), f32(w.vm), dtype, u_hi_t, u_lo_t,
+                           banks, dim, g, n_video, span, rank, f32(w.var), f32(w.cvk_part),
+                           base + w.cvk_t, base + w.w, base + w.kbar, base + w.vbar, words,
+                           (int)space.counters, s));
   CHECK(mark(2));
   CHECK(recap_coarse_tail(q, dtype, batch, heads, dim, q_stride_b, q_stride_h, q_stride_n, rowmap,
                           partition, base + w.kbar, base + w.vbar, base + w.w, u_t, base + w.cvk_t,

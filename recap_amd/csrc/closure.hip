@@ -8,9 +8,14 @@
 //            hi.hi + hi.lo + lo.hi (recap/sparse/closure.py:42-72, first call only)
 // A workgroup handles `group` consecutive video blocks of one bank and writes one
 // [D][D] partial per group; partial_reduce sums the groups in a fixed order and divides
-// by the video token count.  tables builds the query-type tables of the coarse tail
+// by the video token count.  The per-call statistics (rot | cvk) may cut a group into `parts`
+// nearly equal runs of blocks: each run is accumulated from zero and the runs' sums are added in
+// order, by the workgroup that walks the whole group or, with `fine`, by the tables launch over
+// one partial per run, with the same bits.  tables builds the query-type tables of the coarse tail
 // (fold_rank of recap/sparse/closure.py:96-104; kbar, vbar, w casts of
 // recap/kernels/coarse_tail.py:238-241) and basis_tables the U / C_vk casts.
+#include <algorithm>
+
 #include "kernels.hpp"
 
 namespace recap {
@@ -42,8 +47,14 @@ __global__ __launch_bounds__(closure_threads(D, FLAGS), 1) void closure_kernel(C
   __shared__ __attribute__((aligned(16))) float kmean_s[2][D];  // 16-byte copies land here
 
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, g = lane >> 5, l32 = lane & 31;
-  const int bank = blockIdx.x / a.groups, grp = blockIdx.x % a.groups;
-  const int j0 = grp * a.group, j1 = min(j0 + a.group, a.nb);
+  // This workgroup's partial `grp` of its bank: blocks j0 .. j1 - 1, of runs `piece` .. (one with
+  // `fine`) of the group that starts at block g0.
+  const int per_bank = a.fine ? a.groups * a.parts : a.groups;
+  const int bank = blockIdx.x / per_bank, grp = blockIdx.x % per_bank;
+  const int g0 = (a.fine ? grp / a.parts : grp) * a.group, len = min(a.group, a.nb - g0);
+  int piece = a.fine ? grp % a.parts : 0;
+  const int j0 = g0 + len * piece / a.parts;
+  const int j1 = a.fine ? g0 + len * (piece + 1) / a.parts : g0 + len;
   const int rot_tile = SPLIT ? (wave < 4 ? wave : -1) : D == 128 ? wave : (wave < 2 ? wave : -1);
   const int mat_tile = SPLIT ? (wave >= 4 ? wave - 4 : -1)
                              : D == 128 ? wave : (wave >= 2 ? wave - 2 : -1);
@@ -93,10 +104,14 @@ __global__ __launch_bounds__(closure_threads(D, FLAGS), 1) void closure_kernel(C
                     e >> 1 == 3 ? one : 0u};
   }
   f32x16 sacc[SCAT ? NT : 1];
+  f32x16 total[CVK ? NT : 1];  // the finished runs' sums
   if constexpr (CVK) {
     if (mat_tile >= 0) {
 #pragma unroll
-      for (int i = 0; i < NT; ++i) cset(i, f32x16{});
+      for (int i = 0; i < NT; ++i) {
+        cset(i, f32x16{});
+        total[i] = f32x16{};
+      }
     }
   }
 #pragma unroll
@@ -290,7 +305,13 @@ __global__ __launch_bounds__(closure_threads(D, FLAGS), 1) void closure_kernel(C
       }
     }
   };
-  auto mat_work = [&](auto u, const char* ks, const char* vs, int, int count,
+  int run_end = j0;
+  auto next_run = [&](int done) {  // the end of the first run that reaches past block `done`
+    while (run_end <= done && piece < a.parts)
+      run_end = __builtin_amdgcn_readfirstlane(g0 + len * ++piece / a.parts);
+  };
+  next_run(j0);
+  auto mat_work = [&](auto u, const char* ks, const char* vs, int j, int count,
                       const float* kmean_b) {
     constexpr int HF = decltype(u)::value & 1;
     if constexpr (CVK) {
@@ -352,6 +373,16 @@ __global__ __launch_bounds__(closure_threads(D, FLAGS), 1) void closure_kernel(C
               cset(mt, T::mfma32(va[hh][mt], blo[hh], c));
             }
         }
+        if constexpr (HF == 1) {
+          if (j + 1 == run_end) {  // uniform: the run is complete
+#pragma unroll
+            for (int mt = 0; mt < NT; ++mt) {
+              total[mt] += cget(mt);
+              cset(mt, f32x16{});
+            }
+            next_run(j + 1);
+          }
+        }
       }
     }
     if constexpr (SCAT) {
@@ -390,7 +421,7 @@ __global__ __launch_bounds__(closure_threads(D, FLAGS), 1) void closure_kernel(C
   else run(idle);
 
   if (mat_tile >= 0) {
-    const int64_t pbase = ((int64_t)bank * a.groups + grp) * D * D;
+    const int64_t pbase = ((int64_t)bank * per_bank + grp) * D * D;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -399,7 +430,7 @@ __global__ __launch_bounds__(closure_threads(D, FLAGS), 1) void closure_kernel(C
         // columns of tile nt.
         if constexpr (CVK)
           a.cvk_part[pbase + (int64_t)(32 * nt + mfma_row(rr, g)) * D + 32 * mat_tile + l32] =
-              cget(nt)[rr];
+              total[nt][rr];
         if constexpr (SCAT)
           a.scat_part[pbase + (int64_t)(32 * mat_tile + mfma_row(rr, g)) * D + 32 * nt + l32] =
               sacc[nt][rr];
@@ -409,7 +440,7 @@ __global__ __launch_bounds__(closure_threads(D, FLAGS), 1) void closure_kernel(C
 
 template <class T, int D>
 static hipError_t launch_closure(const ClosureArgs& a, int flags, hipStream_t s) {
-  const dim3 grid((unsigned)(a.banks * a.groups));
+  const dim3 grid((unsigned)(a.banks * a.groups * (a.fine ? a.parts : 1)));
   switch (flags) {
     case kRot:
       hipLaunchKernelGGL((closure_kernel<T, D, kRot>), grid, dim3(closure_threads(D, kRot)), 0, s, a);
@@ -430,6 +461,33 @@ static hipError_t launch_closure(const ClosureArgs& a, int flags, hipStream_t s)
 hipError_t run_closure(const ClosureArgs& a, int dtype, int dim, int flags, hipStream_t s) {
   if (dtype == BF16::code) return dim == 128 ? launch_closure<BF16, 128>(a, flags, s) : launch_closure<BF16, 64>(a, flags, s);
   return dim == 128 ? launch_closure<F16, 128>(a, flags, s) : launch_closure<F16, 64>(a, flags, s);
+}
+
+// One round of workgroups (one fits a CU): the fewest rounds that keep at least nine tenths of
+// the 256 CUs busy, so a group is as long as that allows and its prologue (the basis, 64 KB) and
+// partial (64 KB) are paid for once.  Kernel and sum: 97 us with 1,032 groups of 3 blocks (four
+// rounds and a bit) -> 58 with 240 of 13 at 12 heads x 32,760 tokens; 42 -> 26 at 12 x 7,800 (732
+// of 1 -> 252 of 3); 461 -> 402 at 24 x 119,056 (2,808 of 8 -> 240 of 93).  The four runs let a
+// quarter of the layer's heads, called alone, spread over as many workgroups.
+ClosureSpan closure_span(int64_t banks, int64_t nb) {
+  int64_t best = 1;
+  double best_use = 0.0;
+  for (int64_t rounds = 1; rounds <= 4; ++rounds) {
+    const int64_t per_bank = std::min<int64_t>(nb, std::max<int64_t>(1, 256 * rounds / banks));
+    const double use = (double)(banks * per_bank) / (256.0 * (double)rounds);
+    if (use > best_use) {
+      best = per_bank;
+      best_use = use;
+    }
+    if (use >= 0.9 || per_bank == nb) break;
+  }
+  const int group = (int)((nb + best - 1) / best);
+  return {group, std::min(4, group)};
+}
+
+bool closure_fine(int64_t banks, int64_t nb, ClosureSpan span) {
+  const int64_t groups = (nb + span.group - 1) / span.group;
+  return span.parts > 1 && banks * groups <= 128;  // half of the CUs would idle
 }
 
 __global__ __launch_bounds__(256) void partial_reduce_kernel(const float* part, int banks, int groups,
@@ -455,9 +513,9 @@ hipError_t run_partial_reduce(const float* part, int banks, int groups, int elem
 }
 
 // One launch for what lies between the closure statistics and the coarse tail, by block range:
-//   * C_vk (when cvk_part is given): the group partials summed in order, divided and rounded
-//     to the query type, 256 elements a block -- partial_reduce and basis_tables in one pass,
-//     with the same bits.  16 partials are requested at a time: the sum is a serial chain of
+//   * C_vk (when cvk_part is given): the group partials (each the sum of its runs' partials)
+//     summed in order, divided and rounded to the query type, 256 elements a block --
+//     partial_reduce and basis_tables in one pass, with the same bits.  16 partials are requested at a time: the sum is a serial chain of
 //     `groups` loads otherwise (12.9 us for 86 groups).
 //   * the coarse tables, two padded table rows (bank, j), j < ntiles * 32, a block: fold_rank
 //     of the rotated variance (recap/sparse/closure.py:96-104), then w, kbar, vbar rounded to
@@ -476,16 +534,25 @@ __global__ __launch_bounds__(256) void tables_kernel(TablesArgs a) {
   if (blk < cvk_blocks) {
     const int64_t idx = (int64_t)blk * 256 + t;
     const int64_t bank = idx / (D * D), e = idx % (D * D);
-    const float* p = a.cvk_part + bank * a.groups * (int64_t)(D * D) + e;
+    const int n = a.groups * a.runs;   // partials of a bank, `runs` a group
+    const float* p = a.cvk_part + bank * n * (int64_t)(D * D) + e;
     constexpr int kAhead = 16;
-    float acc = p[0];
-    for (int i0 = 1; i0 < a.groups; i0 += kAhead) {
+    float acc = 0.0f, group = 0.0f;
+    int run = 0;
+    for (int i0 = 0; i0 < n; i0 += kAhead) {
       float x[kAhead];
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) x[i] = p[(int64_t)min(i0 + i, a.groups - 1) * (D * D)];
+      for (int i = 0; i < kAhead; ++i) x[i] = p[(int64_t)min(i0 + i, n - 1) * (D * D)];
 #pragma unroll
       for (int i = 0; i < kAhead; ++i)
-        if (i0 + i < a.groups) acc += x[i];
+        if (i0 + i < n) {
+          group += x[i];
+          if (++run == a.runs) {
+            acc += group;
+            group = 0.0f;
+            run = 0;
+          }
+        }
     }
     a.cvk_t[idx] = T::from_f(acc / a.divisor);
     return;

@@ -41,7 +41,13 @@ struct ClosureArgs {
   int banks, nb, tb, n_video, group, groups;
   float* var;                                       // [bank][nb][D]
   float* cvk_part; float* scat_part;                // [bank][groups][D][D]
+  int parts = 1, fine = 0;                          // runs of a group; one partial per run
 };
+// Blocks of a group and its runs for the per-call statistics of a layer of `banks` heads.
+struct ClosureSpan { int group, parts; };
+ClosureSpan closure_span(int64_t banks, int64_t nb);
+// Whether a call of `banks` heads (a part of a layer) gives every run its own workgroup.
+bool closure_fine(int64_t banks, int64_t nb, ClosureSpan span);
 hipError_t run_closure(const ClosureArgs& a, int dtype, int dim, int flags, hipStream_t s);
 hipError_t run_partial_reduce(const float* part, int banks, int groups, int elems, float divisor,
                               float* out, hipStream_t s);
@@ -50,7 +56,7 @@ struct TablesArgs {
   uint16_t* w_t; uint16_t* kbar_t; uint16_t* vbar_t;   // element type of the query
   // Optional: C_vk in the query type from its partials [bank][groups][D][D], and counters to
   // zero for a later launch of the same call.
-  const float* cvk_part; int groups; float divisor; uint16_t* cvk_t;
+  const float* cvk_part; int groups, runs; float divisor; uint16_t* cvk_t;  // runs a group
   unsigned* zero; int zero_words;
 };
 

@@ -46,6 +46,8 @@ class Geometry:
     # Video blocks per closure-statistics workgroup, fixed for a whole layer (the partial
     # sums, and so the rounding, depend on it); None: chosen from the call's banks.
     closure_group: int | None = None
+    # (group, parts) of the per-call statistics, fixed for a whole layer likewise.
+    closure_span: tuple[int, int] | None = None
     # Segments of each long query row of the masked attention, fixed for a whole layer like
     # the group above; None: chosen from the call's banks.
     attn_split: int | None = None
@@ -218,6 +220,42 @@ def closure_group(banks: int, nb: int) -> int:
     """Video blocks per closure workgroup: up to CLOSURE_GROUP, fewer when the call has too
     few blocks to give every CU several workgroups (about 1024 in all)."""
     return max(1, min(CLOSURE_GROUP, (banks * nb) // 1024))
+
+
+@functools.lru_cache(maxsize=256)
+def closure_span(banks: int, n_video: int) -> tuple[int, int]:
+    """Blocks of a C_vk partial and its runs, for a layer of `banks` heads."""
+    group, parts = ctypes.c_int64(), ctypes.c_int64()
+    call("recap_closure_span", banks, n_video, ctypes.byref(group), ctypes.byref(parts))
+    return group.value, parts.value
+
+
+def closure_tables(kv: PackedKV, geo: Geometry, basis: "BasisTables", rank: int):
+    """The per-call statistics and coarse tables with a frozen basis, in two launches:
+    (variance, C_vk in the query type, w, kbar, vbar)."""
+    banks, d = kv.k_means.shape[0], kv.dim
+    dev = kv.k_means.device
+    group, parts = geo.closure_span or closure_span(banks, geo.n_video)
+    width = int(_lib.load().recap_coarse_w_width(dtype_code(kv.dtype), d, int(rank)))
+    if width < 0:
+        raise ValueError(f"closure_tables: invalid dtype/dim/rank ({kv.dtype}, {d}, {rank})")
+    for table in (basis.u_hi_t, basis.u_lo_t):
+        if table.dtype != kv.dtype or table.numel() != banks * d * d:
+            raise ValueError(f"basis table of {table.numel()} {table.dtype} values, expected "
+                             f"{banks * d * d} {kv.dtype}")
+    padded = -(-geo.nb // COARSE_SLOTS) * COARSE_SLOTS
+    partials = int(_lib.load().recap_closure_partials(banks, geo.n_video, group, parts))
+    var = torch.empty(banks, geo.nb, d, dtype=torch.float32, device=dev)
+    part = torch.empty(partials, d, d, dtype=torch.float32, device=dev)
+    cvk_t = torch.empty(banks, d, d, dtype=kv.dtype, device=dev)
+    w, kbar, vbar = (torch.empty(banks, padded, c, dtype=kv.dtype, device=dev)
+                     for c in (width, d, d))
+    call("recap_closure_tables", kv.k_tiles.data_ptr(), kv.vt_tiles.data_ptr(),
+         kv.k_means.data_ptr(), kv.v_means.data_ptr(), dtype_code(kv.dtype),
+         basis.u_hi_t.data_ptr(), basis.u_lo_t.data_ptr(), banks, d, geo.n_tokens, geo.n_video,
+         group, parts, int(rank), var.data_ptr(), part.data_ptr(), cvk_t.data_ptr(),
+         w.data_ptr(), kbar.data_ptr(), vbar.data_ptr(), _stream())
+    return var, cvk_t, w, kbar, vbar
 
 
 def closure_stats(kv: PackedKV, geo: Geometry, flags: int, u_hi_t=None, u_lo_t=None,
@@ -460,7 +498,7 @@ def sparse_call(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rowmap: torch
                 dl: torch.Tensor, glref: torch.Tensor, alpha_override: float | None = None,
                 out: torch.Tensor | None = None, events=None) -> torch.Tensor:
     """A whole corrected sparse call with a frozen basis in one library call and one
-    workspace: kv_pack, closure_stats, the tables, coarse_tail and sparse_merge_attn with
+    workspace: kv_pack, closure_tables, coarse_tail and sparse_merge_attn with
     their outputs bit for bit, in five launches.  ``events``: five timing events recorded
     before the first stage and after pack, closure (with the tables), coarse and attention."""
     b, h, n, d = q.shape
@@ -477,9 +515,9 @@ def sparse_call(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rowmap: torch
     if out is None:
         out = torch.empty(b, h, n, d, dtype=q.dtype, device=q.device)
     code = dtype_code(q.dtype)
-    group = geo.closure_group or closure_group(banks, geo.nb)
+    group, parts = geo.closure_span or closure_span(banks, geo.n_video)
     split = geo.attn_split or attn_split(banks, geo)
-    size = _sparse_call_bytes(code, banks, d, n, geo.n_video, group, rank, split)
+    size = _sparse_call_bytes(code, banks, d, n, geo.n_video, group, parts, rank, split)
     work = torch.empty(size, dtype=torch.uint8, device=q.device)
     handles = None
     if events is not None:
@@ -488,7 +526,7 @@ def sparse_call(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rowmap: torch
         handles = (ctypes.c_void_p * 5)(*(event.cuda_event for event in events))
     call("recap_sparse_call", q.data_ptr(), k.data_ptr(), v.data_ptr(), code, b, h, d,
          *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], rowmap.data_ptr(), n, geo.n_video,
-         float(scale), float(theta), rank, group, tables.u_hi_t.data_ptr(),
+         float(scale), float(theta), rank, group, parts, tables.u_hi_t.data_ptr(),
          tables.u_lo_t.data_ptr(), tables.u_t.data_ptr(), partition.data_ptr(),
          kernel_mask.data_ptr(), det.data_ptr(), dl.data_ptr(), glref.data_ptr(),
          -1.0 if alpha_override is None else float(alpha_override), out.data_ptr(),

@@ -76,7 +76,10 @@ class SparseAttention:
     def coarse_tail_context(self, kv: K.PackedKV, geo: K.Geometry) -> dict:
         """Partition-independent statistics (recap/sparse/attention.py:98-202)."""
         dtype = kv.dtype
-        if self._basis is None:
+        rank = int(self.config.closure_rank)
+        if self._basis is not None:
+            var, cvk_t, w, kbar, vbar = K.closure_tables(kv, geo, self._tables, rank)
+        else:
             _, cvk, scatter = K.closure_stats(kv, geo, _lib.CLOSURE_CVK | _lib.CLOSURE_SCATTER)
             basis = K.symmetric_eigen(scatter)[1]   # symmetrises 0.5 (S + S^T) itself
             split = K.basis_tables(basis, None, dtype, split=True)
@@ -90,14 +93,10 @@ class SparseAttention:
             var = torch.gather(var, 2, idx.expand(-1, var.shape[1], -1)).contiguous()
             self._basis = basis
             self._tables = K.basis_tables(basis, None, dtype, split=True, query=True)
-        else:
-            var, cvk, _ = K.closure_stats(kv, geo, _lib.CLOSURE_ROT | _lib.CLOSURE_CVK,
-                                          self._tables.u_hi_t, self._tables.u_lo_t)
-        cvk_t = K.basis_tables(None, cvk, dtype, cvk_table=True).cvk_t
-        rank = int(self.config.closure_rank)
-        w, kbar, vbar = K.coarse_tables(var, kv, rank)
+            cvk_t = K.basis_tables(None, cvk, dtype, cvk_table=True).cvk_t
+            w, kbar, vbar = K.coarse_tables(var, kv, rank)
         return {"w": w, "kbar": kbar, "vbar": vbar, "u_t": self._tables.u_t, "cvk_t": cvk_t,
-                "rank": rank, "variance": var, "cvk": cvk}
+                "rank": rank, "variance": var}
 
     def coarse_tail_apply(self, q, rowmap, context, partition, geo, scale, glref=None):
         """Coarse tail over the omitted blocks (recap/sparse/attention.py:204-231)."""
@@ -208,6 +207,7 @@ def _layer_geometry(n_tokens: int, n_video: int, banks: int, density: float) -> 
     """A layer's block geometry with the choices that hold for every group of its heads."""
     geo = K.Geometry(n_tokens=n_tokens, n_video=n_video)
     return dataclasses.replace(geo, closure_group=K.closure_group(banks, geo.nb),
+                               closure_span=K.closure_span(banks, n_video),
                                attn_split=K.attn_split(banks, geo, density))
 
 

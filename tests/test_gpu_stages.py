@@ -583,6 +583,47 @@ def test_coarse_tail_extreme_partitions(cuda, name):
     assert m < 2e-3, m
 
 
+@pytest.mark.parametrize("name,dtype", [("tiny", torch.bfloat16),
+                                        ("text-first-ragged", torch.float16),
+                                        ("text-last-d128", torch.bfloat16),
+                                        ("video-ragged-d128", torch.float16)])
+@pytest.mark.parametrize("span", [(1, 1), (3, 2), (5, 4), (64, 4)])
+def test_closure_tables_spans(cuda, name, dtype, span):
+    """C_vk over groups of one to all blocks in one to four runs (empty ones among them): the
+    variances and tables bit for bit those of the separate calls, C_vk within the rounding of
+    one ulp of its type and 1e-5 of its norm (fp32 sums in another order), and the same bits
+    when the banks are called one at a time, where every run has a workgroup of its own."""
+    wl = SMALL[name]
+    print(f"case {name} {dtype} span={span}", flush=True)
+    _, k, v = make_qkv(wl, seed=9, dtype=dtype, device=cuda)
+    k, v = k.repeat(1, 40, 1, 1), v.repeat(1, 40, 1, 1)   # banks enough for one partial a group
+    layout = Layout.from_permutation(hilbert_permutation(wl.grid), text_tokens=wl.text_tokens,
+                                     text_first=wl.text_first)
+    rowmap = layout.rowmap(cuda)
+    geo = K.Geometry(wl.tokens, wl.video_tokens, closure_group=2, closure_span=span)
+    kv = K.kv_pack(k, v, rowmap, geo)
+    banks = k.shape[1]
+    g = torch.Generator().manual_seed(1)
+    basis = torch.linalg.qr(torch.randn(banks, wl.dim, wl.dim, generator=g))[0].to(cuda)
+    tables = K.basis_tables(basis, None, dtype, split=True)
+    var, cvk_t, w, kbar, vbar = K.closure_tables(kv, geo, tables, 4)
+    ref, cvk, _ = K.closure_stats(kv, geo, _lib.CLOSURE_ROT | _lib.CLOSURE_CVK, tables.u_hi_t,
+                                  tables.u_lo_t)
+    assert torch.equal(var, ref)
+    for got, want in zip((w, kbar, vbar), K.coarse_tables(ref, kv, 4)):
+        assert torch.equal(got, want)
+    spread = 1e-5 * cvk.norm() / cvk.numel() ** 0.5
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert bool(((cvk_t.float() - cvk).abs() <= spread + ulp * cvk.abs() + 2.0 ** -24).all())
+    for bank in (0, banks - 1):
+        one = K.kv_pack(k[:, bank:bank + 1], v[:, bank:bank + 1], rowmap, geo)
+        part = K.BasisTables(u_hi_t=tables.u_hi_t[bank:bank + 1].contiguous(),
+                             u_lo_t=tables.u_lo_t[bank:bank + 1].contiguous())
+        alone = K.closure_tables(one, geo, part, 4)
+        for got, want in zip(alone, (var, cvk_t, w, kbar, vbar)):
+            assert torch.equal(got[0], want[bank])
+
+
 @pytest.mark.parametrize("name,dtype,rank,alpha", [
     ("tiny", torch.bfloat16, 4, None),                  # folded w, whole blocks, no text
     ("text-first-ragged", torch.float16, 4, None),      # full-width w, shared ragged block
@@ -599,7 +640,8 @@ def test_sparse_call_equals_its_stages(cuda, name, dtype, rank, alpha):
     layout = Layout.from_permutation(hilbert_permutation(wl.grid), text_tokens=wl.text_tokens,
                                      text_first=wl.text_first)
     rowmap, scale, theta = layout.rowmap(cuda), scale_for(wl.dim), 2.0
-    geo = K.Geometry(wl.tokens, wl.video_tokens, closure_group=2, attn_split=2)
+    geo = K.Geometry(wl.tokens, wl.video_tokens, closure_group=2, closure_span=(2, 1),
+                     attn_split=2)
     kv = K.kv_pack(k, v, rowmap, geo)
     part, kmask = K.pool_select(q, kv.k_means, rowmap, geo, wl.density, scale)
     _, _, scatter = K.closure_stats(kv, geo, _lib.CLOSURE_CVK | _lib.CLOSURE_SCATTER)

@@ -135,28 +135,45 @@ def test_argument_validation_before_launch():
 def test_sparse_call_is_checked_before_any_launch():
     """recap_sparse_call rejects bad sizes, pointers, strides and workspaces on the host."""
     lib = _lib.load()
-    size = lib.recap_sparse_call_workspace_size(_lib.RECAP_BF16, 2, 64, 512, 512, 1, 4, 1)
+    size = lib.recap_sparse_call_workspace_size(_lib.RECAP_BF16, 2, 64, 512, 512, 1, 1, 4, 1)
     assert size > 0
-    for bad in [(9, 2, 64, 512, 512, 1, 4, 1), (_lib.RECAP_BF16, 0, 64, 512, 512, 1, 4, 1),
-                (_lib.RECAP_BF16, 2, 96, 512, 512, 1, 4, 1),
-                (_lib.RECAP_BF16, 2, 64, 500, 512, 1, 4, 1),
-                (_lib.RECAP_BF16, 2, 64, 512, 512, 0, 4, 1),
-                (_lib.RECAP_BF16, 2, 64, 512, 512, 1, 4, 9)]:
+    for bad in [(9, 2, 64, 512, 512, 1, 1, 4, 1), (_lib.RECAP_BF16, 0, 64, 512, 512, 1, 1, 4, 1),
+                (_lib.RECAP_BF16, 2, 96, 512, 512, 1, 1, 4, 1),
+                (_lib.RECAP_BF16, 2, 64, 500, 512, 1, 1, 4, 1),
+                (_lib.RECAP_BF16, 2, 64, 512, 512, 0, 1, 4, 1),
+                (_lib.RECAP_BF16, 2, 64, 512, 512, 1, 0, 4, 1),
+                (_lib.RECAP_BF16, 2, 64, 512, 512, 1, 1, 4, 9)]:
         assert lib.recap_sparse_call_workspace_size(*bad) == -1
     names = ["q", "k", "v", "dtype", "batch", "heads", "dim", "qb", "qh", "qn", "kb", "kh", "kn",
-             "vb", "vh", "vn", "rowmap", "n", "nv", "scale", "theta", "rank", "group", "uh", "ul",
+             "vb", "vh", "vn", "rowmap", "n", "nv", "scale", "theta", "rank", "group", "parts", "uh", "ul",
              "u", "part", "mask", "det", "dl", "ref", "alpha", "out", "ob", "oh", "on", "split",
              "events", "work", "bytes", "stream"]
     good = dict(zip(names, [16, 16, 16, _lib.RECAP_BF16, 1, 2, 64, 0, 0, 64, 0, 0, 64, 0, 0, 64,
-                            16, 512, 512, 0.125, 2.0, 4, 1, 16, 16, 16, 16, 16, 16, 16, 16, -1.0,
+                            16, 512, 512, 0.125, 2.0, 4, 1, 1, 16, 16, 16, 16, 16, 16, 16, 16, -1.0,
                             16, 0, 0, 64, 1, None, 16, size, 0]))
     for name, value in [("k", None), ("v", 8), ("kn", 3), ("out", None), ("rank", 65),
-                        ("rank", -1), ("group", 0), ("split", 9), ("theta", -1.0), ("scale", 0.0),
+                        ("rank", -1), ("group", 0), ("parts", 65), ("split", 9), ("theta", -1.0), ("scale", 0.0),
                         ("u", None), ("uh", 8), ("part", None), ("mask", None), ("det", None),
                         ("ref", None), ("work", None), ("work", 8), ("bytes", size - 1),
                         ("n", 400), ("dim", 80), ("dtype", 7), ("rowmap", None)]:
         with pytest.raises(ValueError):
             _lib.call("recap_sparse_call", *{**good, name: value}.values())
+
+
+@pytest.mark.parametrize("banks", [1, 2, 12, 24, 48, 96, 300])
+@pytest.mark.parametrize("nb", [1, 2, 32, 61, 256, 929, 2048])
+def test_closure_span_rule(banks, nb):
+    """Groups that cover every block, four runs at most, no more than four rounds of
+    workgroups, and partials for a whole layer and for parts of it."""
+    lib = _lib.load()
+    from recap_amd import kernels as K
+    group, parts = K.closure_span(banks, 128 * nb)
+    groups = -(-nb // group)
+    assert 1 <= group <= nb and parts == min(4, group)
+    assert groups * banks <= max(4 * 256, banks)
+    whole = lib.recap_closure_partials(banks, 128 * nb, group, parts)
+    assert whole in (banks * groups, banks * groups * parts)
+    assert lib.recap_closure_partials(banks, 128 * nb, 0, 1) == -1
 
 
 @pytest.mark.parametrize("banks,nt,nv,density", [(12, 4856, 4600, 0.2), (12, 32760, 32760, 0.4),
