@@ -281,6 +281,14 @@ int recap_sparse_merge_attn_ws(const void* q, int dtype, int64_t batch, int64_t 
                                int64_t out_stride_n, int64_t split, int balance,
                                void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The first call's basis and its rotated variances [banks, nb, dim] with the columns in the
+ * order of the pooled within-block variance, largest first, and the tables of
+ * recap_basis_tables for that order; outputs are separate buffers.
+ * Replaces recap/sparse/attention.py:137-152. */
+int recap_order_basis(const float* basis, const float* variance, int dtype, int64_t banks,
+                      int64_t dim, int64_t n_video, float* basis_out, float* variance_out,
+                      void* u_hi_t, void* u_lo_t, void* u_t, void* stream);
+
 /* The per-call closure statistics and the tables of the coarse tail in two launches: the
  * rotated variances (ROT) and C_vk (CVK) of recap_closure_stats, C_vk summed, divided by
  * n_video and rounded to `dtype` (cvk_t [banks, dim, dim]), and the tables of

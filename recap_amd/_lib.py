@@ -57,6 +57,7 @@ SIGNATURES: dict[str, tuple] = {
     "recap_sparse_merge_attn": (_I, [_P, _I, _I64, _I64, _I64, *_STRIDES, _P, _P, _P, _P, _I64,
                                      _I64, _F, _P, _P, _P, _P, _P, _P, _F, _P, *_STRIDES, _P, _P]),
     "recap_attn_queue_words": (_I64, []),
+    "recap_order_basis": (_I, [_P, _P, _I, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P]),
     "recap_closure_span": (_I, [_I64, _I64, _P, _P]),
     "recap_closure_partials": (_I64, [_I64, _I64, _I64, _I64]),
     "recap_closure_tables": (_I, [_P, _P, _P, _P, _I, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64,

@@ -373,6 +373,24 @@ int recap_basis_tables(const float* basis, const float* cvk, int dtype, int64_t 
   return hip_status(run_basis_tables(a, dtype, as_stream(stream)), "basis_tables launch");
 }
 
+int recap_order_basis(const float* basis, const float* variance, int dtype, int64_t banks,
+                      int64_t dim, int64_t n_video, float* basis_out, float* variance_out,
+                      void* u_hi_t, void* u_lo_t, void* u_t, void* stream) {
+  CHECK(check_common(dtype, dim));
+  REQUIRE(basis && variance && basis_out && variance_out && u_hi_t && u_lo_t && u_t, "NULL pointer");
+  REQUIRE(basis != basis_out && variance != variance_out, "outputs must not be the inputs");
+  REQUIRE(banks >= 1, "bad banks");
+  CHECK(check_tokens(n_video, n_video));
+  OrderArgs a{};
+  a.basis = basis; a.var = variance;
+  a.banks = (int)banks; a.dim = (int)dim; a.nb = (int)((n_video + kBlock - 1) / kBlock);
+  a.n_video = (int)n_video;
+  a.basis_out = basis_out; a.var_out = variance_out;
+  a.u_hi_t = static_cast<uint16_t*>(u_hi_t); a.u_lo_t = static_cast<uint16_t*>(u_lo_t);
+  a.u_t = static_cast<uint16_t*>(u_t);
+  return hip_status(run_order_basis(a, dtype, as_stream(stream)), "order_basis launch");
+}
+
 int recap_coarse_tail(const void* q, int dtype, int64_t batch, int64_t heads, int64_t dim,
                       int64_t stride_b, int64_t stride_h, int64_t stride_n,
                       const int32_t* rowmap, const uint8_t* partition, const void* kbar,

@@ -631,6 +631,59 @@ __global__ __launch_bounds__(256) void basis_tables_kernel(BasisArgs a) {
   if (a.cvk_t) a.cvk_t[idx] = T::from_f(a.cvk[idx]);  // C_vk[m][d], row-major
 }
 
+// The first call's basis in the order of the pooled within-block variance, largest first
+// (recap/sparse/attention.py:137-152), with the rotated variances and the query-type tables in
+// that order: one workgroup per bank and one launch, for the pooled sums, their ranks (ties to
+// the lower column, NaN first) and the permuted outputs (20 us at 12 heads x 61 blocks of d = 128,
+// latency; the 15 launches it replaces, a sort among them, took ~60 us and as much of the host).
+constexpr int kOrderThreads = 1024;
+
+template <class T>
+__global__ __launch_bounds__(kOrderThreads) void order_basis_kernel(OrderArgs a) {
+  __shared__ float part[kOrderThreads];
+  __shared__ unsigned key[128];
+  __shared__ int from[128];   // input column of output column o
+  const int D = a.dim, t = threadIdx.x, c = t % D, lanes = kOrderThreads / D;
+  const int64_t bank = blockIdx.x;
+  const float* var = a.var + bank * a.nb * D;
+  float acc = 0.0f;
+  for (int j = t / D; j < a.nb; j += lanes)
+    acc += var[(int64_t)j * D + c] * (float)min(kBlock, a.n_video - kBlock * j);
+  part[t] = acc;
+  __syncthreads();
+  if (t < D) {
+    float sum = part[t];
+    for (int i = 1; i < lanes; ++i) sum += part[t + i * D];
+    const unsigned bits = __float_as_uint(sum / (float)a.n_video);
+    key[t] = sum != sum ? ~0u : ((bits >> 31) ? ~bits : (bits | 0x80000000u));
+  }
+  __syncthreads();
+  if (t < D) {
+    int rank = 0;
+    for (int i = 0; i < D; ++i) rank += key[i] > key[t] || (key[i] == key[t] && i < t);
+    from[rank] = t;
+  }
+  __syncthreads();
+  const float* basis = a.basis + bank * D * D;
+  for (int idx = t; idx < D * D; idx += kOrderThreads) {
+    const int64_t at = bank * D * D + idx;
+    a.basis_out[at] = basis[idx - c + from[c]];          // U[d][from[o]], row-major (idx % D = c)
+    const float u = basis[c * D + from[idx / D]];        // U^T: row o = idx / D, column d = c
+    const uint16_t hi = T::from_f(u);
+    a.u_hi_t[at] = hi;
+    a.u_lo_t[at] = T::from_f(u - T::to_f(hi));
+    a.u_t[at] = hi;
+  }
+  for (int64_t idx = t; idx < (int64_t)a.nb * D; idx += kOrderThreads)
+    a.var_out[bank * a.nb * D + idx] = var[idx - c + from[c]];
+}
+
+hipError_t run_order_basis(const OrderArgs& a, int dtype, hipStream_t s) {
+  if (dtype == BF16::code) hipLaunchKernelGGL(order_basis_kernel<BF16>, dim3((unsigned)a.banks), dim3(kOrderThreads), 0, s, a);
+  else hipLaunchKernelGGL(order_basis_kernel<F16>, dim3((unsigned)a.banks), dim3(kOrderThreads), 0, s, a);
+  return hipGetLastError();
+}
+
 hipError_t run_basis_tables(const BasisArgs& a, int dtype, hipStream_t s) {
   const int64_t total = (int64_t)a.banks * a.dim * a.dim;
   const dim3 grid((unsigned)((total + 255) / 256)), block(256);

@@ -79,6 +79,11 @@ struct BasisArgs {
   uint16_t* u_t; uint16_t* cvk_t;        // U^T and C_vk in the query type (coarse tail)
 };
 hipError_t run_basis_tables(const BasisArgs& a, int dtype, hipStream_t s);
+struct OrderArgs {
+  const float* basis; const float* var; int banks, dim, nb, n_video;   // [bank][D][D], [bank][nb][D]
+  float* basis_out; float* var_out; uint16_t* u_hi_t; uint16_t* u_lo_t; uint16_t* u_t;
+};
+hipError_t run_order_basis(const OrderArgs& a, int dtype, hipStream_t s);
 
 // Symmetric eigen-decomposition of the closure scatter (eigen.hip).
 struct EigenArgs {

@@ -14,53 +14,71 @@
 
 namespace recap {
 
-template <int D>
+// A workgroup computes TILE x TILE scores, (TILE / 16)^2 a thread.  Every score is a chain of
+// D dependent additions, so the smaller tiles trade reuse for workgroups where the larger ones
+// would leave CUs idle: run_block_scores takes the largest tile that gives at least two
+// workgroups a CU (41 -> 22 us at 12 heads x 256 blocks, 33 -> 9 us at 12 x 61; the same bits).
+template <int D, int TILE>
 __global__ __launch_bounds__(256) void block_scores_kernel(ScoreArgs a) {
 #pragma clang fp contract(off)
-  __shared__ float qs[64][D + 1];
-  __shared__ float ks[64][D + 1];
-  const int bank = blockIdx.z, i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
+  constexpr int R = TILE / 16;
+  __shared__ float qs[TILE][D + 1];
+  __shared__ float ks[TILE][D + 1];
+  const int bank = blockIdx.z, i0 = blockIdx.y * TILE, j0 = blockIdx.x * TILE;
   const int t = threadIdx.x;
   const float* qm = a.qm + (int64_t)bank * a.nb * D;
   const float* km = a.km + (int64_t)bank * a.nb * D;
-  for (int idx = t; idx < 64 * D; idx += 256) {
+  for (int idx = t; idx < TILE * D; idx += 256) {
     const int r = idx / D, c = idx % D;
     qs[r][c] = (i0 + r < a.nb) ? qm[(int64_t)(i0 + r) * D + c] : 0.0f;
     ks[r][c] = (j0 + r < a.nb) ? km[(int64_t)(j0 + r) * D + c] : 0.0f;
   }
   __syncthreads();
   const int ty = t >> 4, tx = t & 15;
-  float acc[4][4];
+  float acc[R][R];
 #pragma unroll
-  for (int ai = 0; ai < 4; ++ai)
+  for (int ai = 0; ai < R; ++ai)
 #pragma unroll
-    for (int bj = 0; bj < 4; ++bj) acc[ai][bj] = qs[ty + 16 * ai][0] * ks[tx + 16 * bj][0];
+    for (int bj = 0; bj < R; ++bj) acc[ai][bj] = qs[ty + 16 * ai][0] * ks[tx + 16 * bj][0];
+#pragma unroll 8
   for (int c = 1; c < D; ++c) {
-    float qv[4], kv[4];
+    float qv[R], kv[R];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) { qv[i] = qs[ty + 16 * i][c]; kv[i] = ks[tx + 16 * i][c]; }
+    for (int i = 0; i < R; ++i) { qv[i] = qs[ty + 16 * i][c]; kv[i] = ks[tx + 16 * i][c]; }
 #pragma unroll
-    for (int ai = 0; ai < 4; ++ai)
+    for (int ai = 0; ai < R; ++ai)
 #pragma unroll
-      for (int bj = 0; bj < 4; ++bj) acc[ai][bj] = acc[ai][bj] + qv[ai] * kv[bj];  // two roundings (contract off)
+      for (int bj = 0; bj < R; ++bj) acc[ai][bj] = acc[ai][bj] + qv[ai] * kv[bj];  // two roundings (contract off)
   }
   float* out = a.scores + (int64_t)bank * a.nb * a.nb;
 #pragma unroll
-  for (int ai = 0; ai < 4; ++ai) {
+  for (int ai = 0; ai < R; ++ai) {
     const int i = i0 + ty + 16 * ai;
 #pragma unroll
-    for (int bj = 0; bj < 4; ++bj) {
+    for (int bj = 0; bj < R; ++bj) {
       const int j = j0 + tx + 16 * bj;
       if (i < a.nb && j < a.nb) out[(int64_t)i * a.nb + j] = acc[ai][bj] * a.scale;
     }
   }
 }
 
-hipError_t run_block_scores(const ScoreArgs& a, hipStream_t s) {
-  const dim3 grid((a.nb + 63) / 64, (a.nb + 63) / 64, a.banks), block(256);
-  if (a.dim == 128) hipLaunchKernelGGL(block_scores_kernel<128>, grid, block, 0, s, a);
-  else hipLaunchKernelGGL(block_scores_kernel<64>, grid, block, 0, s, a);
+template <int TILE>
+static hipError_t launch_block_scores(const ScoreArgs& a, hipStream_t s) {
+  const unsigned tiles = (unsigned)((a.nb + TILE - 1) / TILE);
+  const dim3 grid(tiles, tiles, (unsigned)a.banks), block(256);
+  if (a.dim == 128) hipLaunchKernelGGL((block_scores_kernel<128, TILE>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((block_scores_kernel<64, TILE>), grid, block, 0, s, a);
   return hipGetLastError();
+}
+
+hipError_t run_block_scores(const ScoreArgs& a, hipStream_t s) {
+  auto groups = [&](int64_t tile) {
+    const int64_t n = (a.nb + tile - 1) / tile;
+    return n * n * a.banks;
+  };
+  if (groups(64) >= 512) return launch_block_scores<64>(a, s);
+  if (groups(32) >= 512) return launch_block_scores<32>(a, s);
+  return launch_block_scores<16>(a, s);
 }
 
 // Top-k by radix select, one wave per row.  Scores become order-preserving 32-bit keys
@@ -230,12 +248,24 @@ __global__ __launch_bounds__(256) void overlap_partial_kernel(const uint8_t* a, 
   }
 }
 
-__global__ void overlap_final_kernel(unsigned long long* part) {
-  if (threadIdx.x == 0) {
-    unsigned long long k = 0, t = 0;
-    for (int i = 0; i < kOverlapBlocks; ++i) { k += part[2 + 2 * i]; t += part[3 + 2 * i]; }
-    part[0] = k;
-    part[1] = t;
+// One thread a partial pair and a halving tree (integer sums, exact in any order; one thread
+// reading all 512 words took 9-11 us, this 2-6).
+__global__ __launch_bounds__(kOverlapBlocks) void overlap_final_kernel(unsigned long long* part) {
+  __shared__ unsigned long long sk[kOverlapBlocks], st[kOverlapBlocks];
+  const int t = threadIdx.x;
+  sk[t] = part[2 + 2 * t];
+  st[t] = part[3 + 2 * t];
+  __syncthreads();
+  for (int h = kOverlapBlocks / 2; h >= 1; h >>= 1) {
+    if (t < h) {
+      sk[t] += sk[t + h];
+      st[t] += st[t + h];
+    }
+    __syncthreads();
+  }
+  if (t == 0) {
+    part[0] = sk[0];
+    part[1] = st[0];
   }
 }
 
@@ -243,7 +273,7 @@ __global__ void overlap_final_kernel(unsigned long long* part) {
 hipError_t run_mask_overlap(const uint8_t* a, const uint8_t* b, int64_t n, unsigned long long* out,
                             hipStream_t s) {
   hipLaunchKernelGGL(overlap_partial_kernel, dim3(kOverlapBlocks), dim3(256), 0, s, a, b, n, out);
-  hipLaunchKernelGGL(overlap_final_kernel, dim3(1), dim3(64), 0, s, out);
+  hipLaunchKernelGGL(overlap_final_kernel, dim3(1), dim3(kOverlapBlocks), 0, s, out);
   return hipGetLastError();
 }
 

@@ -331,6 +331,21 @@ def basis_tables(basis: torch.Tensor | None, cvk: torch.Tensor | None, dtype: to
     return out
 
 
+def order_basis(basis: torch.Tensor, var: torch.Tensor, geo: Geometry, dtype: torch.dtype):
+    """(basis, variances, tables) with the columns in the order of the pooled within-block
+    variance, largest first."""
+    banks, nb, d = var.shape
+    if basis.shape != (banks, d, d) or nb != geo.nb:
+        raise ValueError(f"basis {tuple(basis.shape)} and variances {tuple(var.shape)} do not match")
+    basis, var = basis.contiguous(), var.contiguous()
+    basis_out, var_out = torch.empty_like(basis), torch.empty_like(var)
+    hi, lo, u_t = (torch.empty(banks, d, d, dtype=dtype, device=var.device) for _ in range(3))
+    call("recap_order_basis", basis.data_ptr(), var.data_ptr(), dtype_code(dtype), banks, d,
+         geo.n_video, basis_out.data_ptr(), var_out.data_ptr(), hi.data_ptr(), lo.data_ptr(),
+         u_t.data_ptr(), _stream())
+    return basis_out, var_out, BasisTables(u_hi_t=hi, u_lo_t=lo, u_t=u_t)
+
+
 COARSE_SLOTS = 32  # key blocks per coarse-tail table tile
 
 

@@ -85,14 +85,7 @@ class SparseAttention:
             split = K.basis_tables(basis, None, dtype, split=True)
             var, _, _ = K.closure_stats(kv, geo, _lib.CLOSURE_ROT, split.u_hi_t, split.u_lo_t)
             # Order the basis by pooled within-block variance (recap/sparse/attention.py:137-152).
-            weights = geo.counts(var.device).reshape(1, -1, 1)
-            pooled = (var * weights).sum(1) / weights.sum().clamp_min(1.0)
-            order = torch.argsort(pooled, dim=-1, descending=True)
-            idx = order.unsqueeze(1)
-            basis = torch.gather(basis, 2, idx.expand(-1, basis.shape[1], -1)).contiguous()
-            var = torch.gather(var, 2, idx.expand(-1, var.shape[1], -1)).contiguous()
-            self._basis = basis
-            self._tables = K.basis_tables(basis, None, dtype, split=True, query=True)
+            self._basis, var, self._tables = K.order_basis(basis, var, geo, dtype)
             cvk_t = K.basis_tables(None, cvk, dtype, cvk_table=True).cvk_t
             w, kbar, vbar = K.coarse_tables(var, kv, rank)
         return {"w": w, "kbar": kbar, "vbar": vbar, "u_t": self._tables.u_t, "cvk_t": cvk_t,

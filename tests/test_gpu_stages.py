@@ -583,6 +583,44 @@ def test_coarse_tail_extreme_partitions(cuda, name):
     assert m < 2e-3, m
 
 
+@pytest.mark.parametrize("d,dtype,n_video", [(64, torch.bfloat16, 100), (64, torch.float16, 1300),
+                                             (128, torch.bfloat16, 4096),
+                                             (128, torch.float16, 2500)])
+def test_order_basis(cuda, d, dtype, n_video):
+    """The ordered basis, variances and tables against torch's sort of the pooled variance
+    (well separated columns, and a pair of equal ones that keeps its order)."""
+    banks, geo = 3, K.Geometry(n_video, n_video)
+    g = torch.Generator().manual_seed(d + n_video)
+    basis = torch.randn(banks, d, d, generator=g)
+    scale = torch.stack([torch.randperm(d, generator=g) + 1.0 for _ in range(banks)])
+    var = (1.0 + 0.001 * torch.rand(banks, geo.nb, d, generator=g)) * scale.unsqueeze(1)
+    var[:, :, 5] = var[:, :, 9]
+    counts = geo.counts("cpu").view(1, -1, 1)
+    pooled = (var.double() * counts).sum(1) / n_video
+    order = torch.argsort(pooled, dim=-1, descending=True, stable=True).unsqueeze(1)
+    got, got_var, tables = K.order_basis(basis.to(cuda), var.to(cuda), geo, dtype)
+    want = torch.gather(basis, 2, order.expand(-1, d, -1)).to(cuda)
+    assert torch.equal(got, want)
+    assert torch.equal(got_var.cpu(), torch.gather(var, 2, order.expand(-1, geo.nb, -1)))
+    ref = K.basis_tables(want, None, dtype, split=True, query=True)
+    for name in ("u_hi_t", "u_lo_t", "u_t"):
+        assert torch.equal(getattr(tables, name), getattr(ref, name))
+
+
+@pytest.mark.parametrize("banks,nb,d", [(1, 1, 64), (2, 17, 128), (12, 61, 128), (3, 100, 64),
+                                        (5, 333, 64), (2, 1100, 128)])
+def test_block_scores_tiles(cuda, banks, nb, d):
+    """Every tile size of the scores (16, 32 and 64, by the number of workgroups) against the
+    sequential sum of separately rounded products, bit for bit."""
+    g = torch.Generator().manual_seed(nb)
+    qm, km = (torch.randn(banks, nb, d, generator=g).to(cuda) for _ in range(2))
+    got = K.block_scores(qm, km, 0.3)
+    acc = qm[:, :, None, 0] * km[:, None, :, 0]
+    for c in range(1, d):
+        acc = acc + qm[:, :, None, c] * km[:, None, :, c]
+    assert torch.equal(got, acc * torch.tensor(0.3, dtype=torch.float32, device=cuda))
+
+
 @pytest.mark.parametrize("name,dtype", [("tiny", torch.bfloat16),
                                         ("text-first-ragged", torch.float16),
                                         ("text-last-d128", torch.bfloat16),
