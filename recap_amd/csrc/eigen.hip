@@ -209,16 +209,18 @@ __global__ __launch_bounds__(kEigenThreads) void symmetric_eigen_kernel(EigenArg
 }
 
 // The rotation that zeroes a_pq (alg. 8.5.1): t = tan(theta) of the smaller angle; c = 1 and
-// s = 0 for an entry that is small already.
+// s = 0 for an entry that is small already.  Branch-free, so that the test's chain of operations
+// and the rotation's run side by side (a two-layer schedule with two 4 x 64 decompositions: 2040 ->
+// 1973 us; at 128 no difference); a rotation that is not taken may divide by zero, and its result
+// is dropped.
 __device__ __forceinline__ bool jacobi_rotation(float app, float aqq, float apq, float& c, float& s) {
-  c = 1.0f;
-  s = 0.0f;
-  if (!(fabsf(apq) > kEigenTol * sqrtf(fabsf(app * aqq)) && apq != 0.0f)) return false;
+  const bool turn = fabsf(apq) > kEigenTol * sqrtf(fabsf(app * aqq)) && apq != 0.0f;
   const float tau = (aqq - app) / (2.0f * apq);
   const float tn = copysignf(1.0f, tau) / (fabsf(tau) + sqrtf(1.0f + tau * tau));
-  c = 1.0f / sqrtf(1.0f + tn * tn);
-  s = tn * c;
-  return true;
+  const float ct = 1.0f / sqrtf(1.0f + tn * tn);
+  c = turn ? ct : 1.0f;
+  s = turn ? tn * ct : 0.0f;
+  return turn;
 }
 
 // The same sweeps for n = N = 64 or 128 (the head dimensions) with A and V in registers, bit
