@@ -5,8 +5,8 @@
 //                     (recap/sparse/closure.py:75-81).
 //
 // One workgroup per matrix; the matrix and the accumulated rotations live in registers at the
-// head dimensions 64 and 128, in LDS (2 x 64 KB) at other orders.  Two-sided cyclic Jacobi (Golub & Van Loan, Matrix Computations, 4th ed.,
-// alg. 8.5.2 with the symmetric 2x2 Schur rotation of alg. 8.5.1) in the parallel
+// head dimensions 64 and 128, in LDS (2 x 64 KB) at other orders.  Two-sided cyclic Jacobi
+// (Golub & Van Loan, Matrix Computations, 4th ed., alg. 8.5.2 with the symmetric 2x2 Schur rotation of alg. 8.5.1) in the parallel
 // round-robin ordering of Brent & Luk (1985): a sweep is m - 1 rounds (m = n rounded up
 // to even) of m/2 disjoint index pairs, rotated at once.  In LDS a round is two barriers: the m/2
 // threads that own a pair compute its rotation and publish it with the pair, then every
@@ -234,7 +234,7 @@ __device__ __forceinline__ bool jacobi_rotation(float app, float aqq, float apq,
 // and V's rotations 190, the row moves 85, the rotation itself with its IEEE divisions and
 // roots 75), two waves a SIMD at N = 128, 1.65 us a round.  The kernel above moves both matrices
 // through LDS, 256 KB a round, behind two barriers: 3.84 ms for 12 matrices of order 128 and
-// 1.05 ms for 4 of order 64; here 1.92 and 0.57 ms.
+// 1.05 ms for 4 of order 64; here 1.91 and 0.53 ms.
 template <int N>
 __global__ __launch_bounds__(4 * N) void symmetric_eigen_ring_kernel(EigenArgs a) {
   constexpr int SLOTS = N / 2, P = 8, NW = SLOTS / P, E = N / 64, THREADS = 64 * NW;
