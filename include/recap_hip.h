@@ -254,10 +254,11 @@ int64_t recap_attn_queue_words(void);
  * (the text rows and a ragged last video block, from query block ds on) cut into `split`
  * segments of its kept blocks, which separate workgroups walk and the last of them combines
  * in segment order.  Rows below the long ones are bit-identical to those of the launches
- * without a workspace; a long row's equal them for split 1 and otherwise differ by the
- * rounding of another summation order, the same on every run.  recap_attn_split gives the
- * split for a layer of `banks` heads whose other rows keep about `density` of their blocks
- * (1: none); recap_attn_workspace_size the bytes (16-byte aligned device memory, contents
+ * without a workspace; a long row's equal them for split 1 and otherwise differ by the rounding
+ * of another order of the fp32 sums (where a segment's scores make it raise the running max
+ * again, also by that of P relative to another max), the same on every run.  recap_attn_split
+ * gives the split for a layer of `banks` heads whose other rows keep about `density` of their
+ * blocks (1: none); recap_attn_workspace_size the bytes (16-byte aligned device memory, contents
  * ignored; the counters are zeroed on `stream`).  Calls that may overlap need separate
  * workspaces.  No counterpart in the reference. */
 int64_t recap_attn_split(int64_t banks, int64_t n_tokens, int64_t n_video, double density);

@@ -28,7 +28,8 @@
 // The masked modes walk their kept blocks in one order (a kept ragged last block first,
 // then ascending), and dense-head stores its head branch before the first block after the
 // kept ones can move the running max, so the head branch of head, dense-head and merge
-// modes is the same bit for bit.
+// modes is the same bit for bit; a long row that head or merge mode walks in segments (below)
+// differs from it by the order of its sums.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -487,6 +488,9 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
     if constexpr (D != 64) copy(vrs, image(0), v_lds0);   // (at d = 64 its step copies it)
   }
   if (nsub > 1) copy(krs, image(1), k_lds1);
+  // A later segment also gets the K image of the whole row's first sub-tile (see below).
+  if (kSplits && seg > 0 && nsub > 0)
+    copy(krs, __builtin_amdgcn_readfirstlane(list[0] * G::kTileBytes), v_lds1);
   tile_barrier();
 
   float m[kGroups], mraw[kGroups], lsum[kGroups];
@@ -760,10 +764,22 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
 
   f32x16 sa[kGroups][2], sb[kGroups][2];
   if (nsub > 0) {
+    if (kSplits && seg > 0) {
+      // Every segment of a long row starts from the running max that the undivided walk has
+      // after its first sub-tile: the probabilities, which are rounded to 16 bits relative to
+      // it, are then the undivided walk's (but where a segment's scores make it raise the max
+      // again), and only the order of the fp32 sums is another.  From a
+      // max of their own, 9-34% of the long rows' elements came out as the neighbouring value
+      // (12 heads x 7,800 tokens; 12 x 4,856 in fp16), now 0.8-7%; no time to be seen (127.9
+      // us a sparse call at the second, 128.8 before, runs 2.5% apart).
+      qk(v_lds1, sa);
+      if (ragged && __builtin_amdgcn_readfirstlane(list[0]) == a.tb - 1) mask_tail(sa, 0);
+      row_max(sa);
+    }
     qk(k_lds0, sa);
     if (ragged_at(0)) mask_tail(sa, 0);
     row_max(sa);
-    tile_barrier();  // step 0 overwrites K slot 0 (read just now)
+    tile_barrier();  // the first steps overwrite K slot 0 and V slot 1 (read just now)
   }
   using F = std::false_type;
   using Tr = std::true_type;
