@@ -432,6 +432,9 @@ def _attn_workspace(q: torch.Tensor, geo: Geometry) -> tuple[int, torch.Tensor]:
     b, h, _, d = q.shape
     split = geo.attn_split or attn_split(b * h, geo)
     size = _attn_bytes(b * h, d, geo.n_tokens, geo.n_video, split)
+    if size < 0:
+        raise ValueError(f"invalid attention sizes ({geo.n_tokens} tokens, {geo.n_video} video, "
+                         f"{d}, split {split})")
     return split, torch.empty(size, dtype=torch.uint8, device=q.device)
 
 
@@ -502,6 +505,9 @@ def sparse_merge_attn(q: torch.Tensor, kv: PackedKV, rowmap: torch.Tensor,
     return out
 
 
+_MASKS, _HALF, _FLOAT = (torch.bool, torch.uint8), (torch.float16,), (torch.float32,)
+
+
 @functools.lru_cache(maxsize=256)
 def _sparse_call_bytes(*sizes: int) -> int:
     return int(_lib.load().recap_sparse_call_workspace_size(*sizes))
@@ -516,7 +522,11 @@ def sparse_call(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rowmap: torch
     workspace: kv_pack, closure_tables, coarse_tail and sparse_merge_attn with
     their outputs bit for bit, in five launches.  ``events``: five timing events recorded
     before the first stage and after pack, closure (with the tables), coarse and attention."""
+    if not q.shape == k.shape == v.shape or not q.dtype == k.dtype == v.dtype:
+        raise ValueError("Q, K and V must have the same shape and dtype")
     b, h, n, d = q.shape
+    if n != geo.n_tokens:
+        raise ValueError(f"Q has {n} tokens, the geometry {geo.n_tokens}")
     banks = b * h
     for name in ("u_hi_t", "u_lo_t", "u_t"):
         table = getattr(tables, name)
@@ -524,6 +534,14 @@ def sparse_call(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rowmap: torch
             raise ValueError(f"coarse_tail: table {name} is {table.dtype}, Q is {q.dtype}")
         if table.numel() != banks * d * d:
             raise ValueError(f"table {name} has {table.numel()} elements, expected {banks * d * d}")
+    rows = banks * geo.rows
+    for name, t, size, types in (("partition", partition, banks * geo.nb ** 2, _MASKS),
+                                 ("kernel_mask", kernel_mask, banks * geo.tb ** 2, _MASKS),
+                                 ("det", det, rows * d, _HALF), ("dl", dl, rows, _FLOAT),
+                                 ("glref", glref, rows, _FLOAT)):
+        if t.numel() != size or t.dtype not in types:
+            raise ValueError(f"{name} has {t.numel()} {t.dtype} elements, expected {size} of "
+                             f"{types[0]}")
     partition, kernel_mask = partition.contiguous(), kernel_mask.contiguous()
     if not (det.is_contiguous() and dl.is_contiguous() and glref.is_contiguous()):
         raise ValueError("merge inputs must be contiguous")
@@ -533,6 +551,9 @@ def sparse_call(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rowmap: torch
     group, parts = geo.closure_span or closure_span(banks, geo.n_video)
     split = geo.attn_split or attn_split(banks, geo)
     size = _sparse_call_bytes(code, banks, d, n, geo.n_video, group, parts, rank, split)
+    if size < 0:
+        raise ValueError(f"sparse_call: invalid sizes ({n} tokens, {geo.n_video} video, {d}, rank "
+                         f"{rank}, group {group}, parts {parts}, split {split})")
     work = torch.empty(size, dtype=torch.uint8, device=q.device)
     handles = None
     if events is not None:

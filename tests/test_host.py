@@ -431,3 +431,35 @@ def test_operator_rejects_mixed_qkv_dtypes():
     tables = {n: torch.empty(0, dtype=torch.float16) for n in ("kbar", "vbar", "w", "u_t", "cvk_t")}
     with pytest.raises(ValueError, match="table kbar"):
         K.coarse_tail(q, None, torch.empty(0), None, tables, 0.125, 2.0)
+
+
+@pytest.mark.parametrize("name,change", [
+    ("K and V", dict(k=torch.zeros(1, 2, 256, 64, dtype=torch.bfloat16))),     # another length
+    ("K and V", dict(v=torch.zeros(1, 1, 300, 64, dtype=torch.bfloat16))),     # other heads
+    ("K and V", dict(k=torch.zeros(1, 2, 300, 64, dtype=torch.float16))),      # another type
+    ("tokens", dict(geo=K.Geometry(428, 300))),
+    ("table u_lo_t", dict(tables=K.BasisTables(*(torch.zeros(2, 64, w, dtype=torch.bfloat16)
+                                                 for w in (64, 32, 64))))),
+    ("partition", dict(partition=torch.ones(2, 2, 3, dtype=torch.bool))),
+    ("partition", dict(partition=torch.ones(2, 3, 3))),
+    ("kernel_mask", dict(kernel_mask=torch.ones(1, 3, 3, dtype=torch.bool))),
+    ("det", dict(det=torch.zeros(2, 128, 64, dtype=torch.float16))),
+    ("det", dict(det=torch.zeros(2, 256, 64, dtype=torch.bfloat16))),
+    ("dl", dict(dl=torch.zeros(2, 300))),
+    ("glref", dict(glref=torch.zeros(2, 256, dtype=torch.float16))),
+    ("rank -1", dict(rank=-1)),
+    ("split 9", dict(geo=K.Geometry(300, 300, closure_span=(1, 1), attn_split=9)))])
+def test_sparse_call_wrapper_checks_its_tensors(name, change):
+    """kernels.sparse_call refuses K/V unlike Q (as kv_pack does), tables, masks and bank
+    tensors of another size or type, and sizes without a workspace, before any launch."""
+    q, k, v = (torch.zeros(1, 2, 300, 64, dtype=torch.bfloat16) for _ in range(3))
+    good = dict(q=q, k=k, v=v, rowmap=torch.arange(300, dtype=torch.int32),
+                geo=K.Geometry(300, 300), scale=0.125, theta=2.0, rank=4,
+                tables=K.BasisTables(*(torch.zeros(2, 64, 64, dtype=torch.bfloat16)
+                                       for _ in range(3))),
+                partition=torch.ones(2, 3, 3, dtype=torch.bool),
+                kernel_mask=torch.ones(2, 3, 3, dtype=torch.bool),
+                det=torch.zeros(2, 256, 64, dtype=torch.float16), dl=torch.zeros(2, 256),
+                glref=torch.zeros(2, 256))
+    with pytest.raises(ValueError, match=name):
+        K.sparse_call(**{**good, **change})
