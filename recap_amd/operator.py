@@ -475,28 +475,39 @@ class Operator:
         b, h, n, d = q.shape
         banks = b * h
         scale = K.scale_for(d)
+        events = None
+        if self.stage_events is not None:
+            events = [torch.cuda.Event(enable_timing=True) for _ in _STAGES]
+            for name, event in zip(_STAGES, events):
+                self.stage_events.setdefault(name, []).append(event)
         if layer.frozen:
-            events = None
-            if self.stage_events is not None:
-                events = [torch.cuda.Event(enable_timing=True) for _ in _STAGES]
-                for name, event in zip(_STAGES, events):
-                    self.stage_events.setdefault(name, []).append(event)
             return K.sparse_call(
                 q, k, v, rowmap, geo, scale, self.config.closure_gate_theta,
                 int(self.config.closure_rank), layer.tables,
                 bank.partition.reshape(banks, geo.nb, geo.nb), bank.head_kernel_mask, bank.value,
                 bank.log_mass, bank.coarse_lse, self.alpha_override, out, events)
+
         # No basis yet (a bank that was handed in): stage by stage, the basis from these keys.
+        def mark(stage: str) -> None:
+            if events is not None:
+                events[_STAGES.index(stage)].record()
+
+        mark("start")
         kv = K.kv_pack(k, v, rowmap, geo)
+        mark("pack")
         context = layer.coarse_tail_context(kv, geo)
+        mark("closure")
         old_lse = bank.coarse_lse
         go, gl, drift_part = layer.coarse_tail_apply(
             q, rowmap, context, bank.partition.reshape(banks, geo.nb, geo.nb), geo, scale,
             glref=old_lse)
         center = K.drift_center(drift_part, geo) if geo.rows else None
-        return K.sparse_merge_attn(q, kv, rowmap, bank.head_kernel_mask, geo, scale, go, gl,
-                                   bank.value, bank.log_mass, old_lse, center,
-                                   alpha_override=self.alpha_override, out=out)
+        mark("coarse")
+        out = K.sparse_merge_attn(q, kv, rowmap, bank.head_kernel_mask, geo, scale, go, gl,
+                                  bank.value, bank.log_mass, old_lse, center,
+                                  alpha_override=self.alpha_override, out=out)
+        mark("attention")
+        return out
 
     # -- the refinement error ------------------------------------------------------------
 

@@ -338,6 +338,39 @@ def test_hunyuan_bank_chunks_and_host_banks_are_identical(hunyuan_inputs):
             assert torch.equal(a, b), label
 
 
+@pytest.mark.parametrize("name", ["text-first-ragged", "text-last-d128"])
+def test_sparse_call_on_a_bank_handed_in(cuda, name):
+    """A SPARSE call of an operator that was given another one's bank and has no basis yet
+    takes it from its own keys, stage by stage: with the keys of the other's refresh that is
+    the same basis, and the output is the other's SPARSE output but for the order in which
+    C_vk is summed.  Both routes record every stage event once a call."""
+    wl = SMALL[name]
+    print(f"case {name}", flush=True)
+    q, k, v = (x.to(cuda) for x in make_qkv(wl, seed=0))
+    outs, ops = [], []
+    for _ in range(2):
+        op, _ = build(wl, layers=1)
+        op.stage_events = {}
+        if ops:
+            op.banks[0][0] = ops[0].banks[0][0]
+        else:
+            op.begin_step(0, REFRESH)
+            op.attend(0, q, k, v)
+        op.begin_step(1, SPARSE)
+        assert op.layers[0][0].frozen != bool(ops)
+        outs.append(op.attend(0, q, k, v))
+        ops.append(op)
+    torch.cuda.synchronize()
+    assert torch.equal(ops[0].layers[0][0].basis, ops[1].layers[0][0].basis)
+    assert_parity(outs[1].float(), outs[0].float(), f"handed-in bank {name}")
+    for op in ops:
+        events = op.stage_events
+        assert list(events) == ["start", "pack", "closure", "coarse", "attention"]
+        assert all(len(e) == 1 for e in events.values())
+        times = [events["start"][0].elapsed_time(e[0]) for e in events.values()]
+        assert times == sorted(times) and times[-1] > 0.0, times
+
+
 @pytest.mark.parametrize("name", ["wan2.1-480p", "hunyuan-720p"])
 def test_work_queue_schedule_gives_identical_outputs(cuda, monkeypatch, name):
     """The attention launches with per-XCD claim queues (XCDs that finish early take the
