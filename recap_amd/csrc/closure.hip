@@ -15,6 +15,7 @@
 // (fold_rank of recap/sparse/closure.py:96-104; kbar, vbar, w casts of
 // recap/kernels/coarse_tail.py:238-241) and basis_tables the U / C_vk casts.
 #include <algorithm>
+#include <cstdint>
 
 #include "kernels.hpp"
 
@@ -468,18 +469,34 @@ hipError_t run_closure(const ClosureArgs& a, int dtype, int dim, int flags, hipS
 // partial (64 KB) are paid for once.  Kernel and sum: 97 us with 1,032 groups of 3 blocks (four
 // rounds and a bit) -> 58 with 240 of 13 at 12 heads x 32,760 tokens; 42 -> 26 at 12 x 7,800 (732
 // of 1 -> 252 of 3); 461 -> 402 at 24 x 119,056 (2,808 of 8 -> 240 of 93).  The four runs let a
-// quarter of the layer's heads, called alone, spread over as many workgroups.
+// quarter of the layer's heads, called alone, spread over as many workgroups.  More than 256 banks
+// take several rounds whatever the group, and one group a bank would leave the last of them nearly
+// empty (closure and tables 274 us at 300 banks of 61 blocks, d = 64, now 202; 1,111 -> 726 at 300
+// of 256): there the group is the one with the shortest rounds, a workgroup's prologue and
+// partial counted as two blocks (by the figures above).
 ClosureSpan closure_span(int64_t banks, int64_t nb) {
   int64_t best = 1;
-  double best_use = 0.0;
-  for (int64_t rounds = 1; rounds <= 4; ++rounds) {
-    const int64_t per_bank = std::min<int64_t>(nb, std::max<int64_t>(1, 256 * rounds / banks));
-    const double use = (double)(banks * per_bank) / (256.0 * (double)rounds);
-    if (use > best_use) {
-      best = per_bank;
-      best_use = use;
+  if (banks > 256) {
+    int64_t least = INT64_MAX;
+    for (int64_t per_bank = 1; per_bank <= std::min<int64_t>(nb, 32); ++per_bank) {
+      const int64_t group = (nb + per_bank - 1) / per_bank, groups = (nb + group - 1) / group;
+      const int64_t time = (banks * groups + 255) / 256 * (group + 2);
+      if (time < least) {
+        best = per_bank;
+        least = time;
+      }
     }
-    if (use >= 0.9 || per_bank == nb) break;
+  } else {
+    double best_use = 0.0;
+    for (int64_t rounds = 1; rounds <= 4; ++rounds) {
+      const int64_t per_bank = std::min<int64_t>(nb, 256 * rounds / banks);
+      const double use = (double)(banks * per_bank) / (256.0 * (double)rounds);
+      if (use > best_use) {
+        best = per_bank;
+        best_use = use;
+      }
+      if (use >= 0.9 || per_bank == nb) break;
+    }
   }
   const int group = (int)((nb + best - 1) / best);
   return {group, std::min(4, group)};

@@ -160,17 +160,24 @@ def test_sparse_call_is_checked_before_any_launch():
             _lib.call("recap_sparse_call", *{**good, name: value}.values())
 
 
-@pytest.mark.parametrize("banks", [1, 2, 12, 24, 48, 96, 300])
+@pytest.mark.parametrize("banks", [1, 2, 12, 24, 48, 96, 255, 257, 300, 384, 511, 513, 1000])
 @pytest.mark.parametrize("nb", [1, 2, 32, 61, 256, 929, 2048])
 def test_closure_span_rule(banks, nb):
-    """Groups that cover every block, four runs at most, no more than four rounds of
-    workgroups, and partials for a whole layer and for parts of it."""
+    """Groups that cover every block, four runs at most, no more than four rounds of workgroups
+    up to 256 banks, and partials for a whole layer and for parts of it.  Above 256 banks, where
+    the last round may be nearly empty, the launch is no longer than with groups of eight blocks
+    or with one a bank, by the time of a workgroup (its blocks and a prologue worth two)."""
     lib = _lib.load()
     from recap_amd import kernels as K
     group, parts = K.closure_span(banks, 128 * nb)
     groups = -(-nb // group)
     assert 1 <= group <= nb and parts == min(4, group)
-    assert groups * banks <= max(4 * 256, banks)
+    rounds = lambda g: -(-banks * -(-nb // g) // 256)  # noqa: E731
+    if banks <= 256:
+        assert rounds(group) <= 4
+    else:
+        for other in (K.closure_group(banks, nb), nb):
+            assert rounds(group) * (group + 2) <= 1.1 * rounds(other) * (other + 2), other
     whole = lib.recap_closure_partials(banks, 128 * nb, group, parts)
     assert whole in (banks * groups, banks * groups * parts)
     assert lib.recap_closure_partials(banks, 128 * nb, 0, 1) == -1
