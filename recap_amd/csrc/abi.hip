@@ -683,7 +683,7 @@ static int closure_and_tables(const void* k_tiles, const void* vt_tiles, const f
 }
 
 static int check_span(int64_t group, int64_t parts) {
-  REQUIRE(group >= 1 && group <= 4096 && parts >= 1 && parts <= 64, "bad closure group %lld / parts %lld",
+  REQUIRE(group >= 1 && group <= 4096 && parts >= 1 && parts <= kMaxParts, "bad closure group %lld / parts %lld",
           (long long)group, (long long)parts);
   return RECAP_OK;
 }

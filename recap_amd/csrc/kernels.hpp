@@ -45,6 +45,7 @@ struct ClosureArgs {
 };
 // Blocks of a group and its runs for the per-call statistics of a layer of `banks` heads.
 struct ClosureSpan { int group, parts; };
+constexpr int kMaxParts = 64;
 ClosureSpan closure_span(int64_t banks, int64_t nb);
 // Whether a call of `banks` heads (a part of a layer) gives every run its own workgroup.
 bool closure_fine(int64_t banks, int64_t nb, ClosureSpan span);

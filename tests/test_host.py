@@ -163,15 +163,17 @@ def test_sparse_call_is_checked_before_any_launch():
 @pytest.mark.parametrize("banks", [1, 2, 12, 24, 48, 96, 255, 257, 300, 384, 511, 513, 1000])
 @pytest.mark.parametrize("nb", [1, 2, 32, 61, 256, 929, 2048])
 def test_closure_span_rule(banks, nb):
-    """Groups that cover every block, four runs at most, no more than four rounds of workgroups
-    up to 256 banks, and partials for a whole layer and for parts of it.  Above 256 banks, where
+    """Groups that cover every block, four runs or as many as keep each to 24 blocks (32 in the
+    longest groups: 64 runs at most), no more than four rounds of workgroups up to 256 banks, and
+    partials for a whole layer and for parts of it.  Above 256 banks, where
     the last round may be nearly empty, the launch is no longer than with groups of eight blocks
     or with one a bank, by the time of a workgroup (its blocks and a prologue worth two)."""
     lib = _lib.load()
     from recap_amd import kernels as K
     group, parts = K.closure_span(banks, 128 * nb)
     groups = -(-nb // group)
-    assert 1 <= group <= nb and parts == min(4, group)
+    assert 1 <= group <= nb and parts == min(group, max(4, -(-group // 24)), 64)
+    assert -(-group // parts) <= (24 if group <= 24 * 64 else 32)
     rounds = lambda g: -(-banks * -(-nb // g) // 256)  # noqa: E731
     if banks <= 256:
         assert rounds(group) <= 4
