@@ -375,28 +375,42 @@ def test_sparse_call_on_a_bank_handed_in(cuda, name):
 def test_work_queue_schedule_gives_identical_outputs(cuda, monkeypatch, name):
     """The attention launches with per-XCD claim queues (XCDs that finish early take the
     others' last query blocks) and with the static assignment give bit-identical refresh
-    and sparse outputs: only which workgroup computes a query block changes."""
+    and sparse outputs: only which workgroup computes a query block changes.  The SPARSE call
+    always claims its items, so it is compared with its stages on the operator's own bank and
+    geometry, the merge launch of which runs either way."""
     from recap_amd import kernels as K
     wl = WORKLOADS[name]
     print(f"case {name}", flush=True)
     q, k, v = make_qkv(wl, seed=0, device=cuda)
     q1, k1, v1 = (perturb(x, 0.02, seed=i, step=1) for i, x in enumerate((q, k, v)))
-    outs = {}
-    dense_head, merge = K.dense_head_attn, K.sparse_merge_attn
+    dense, ran = {}, []
+    dense_head = K.dense_head_attn
     for balance in (True, False):
-        monkeypatch.setattr(K, "dense_head_attn",
-                            lambda *a, **kw: dense_head(*a, **kw, balance=balance))
-        monkeypatch.setattr(K, "sparse_merge_attn",
-                            lambda *a, **kw: merge(*a, **kw, balance=balance))
+        def patched(*a, balance=balance, **kw):
+            ran.append(balance)
+            return dense_head(*a, **kw, balance=balance)
+
+        monkeypatch.setattr(K, "dense_head_attn", patched)
         op, _ = build(wl, layers=1)
         op.begin_step(0, REFRESH)
-        dense = op.attend(0, q, k, v).clone()
-        op.begin_step(1, SPARSE)
-        sparse = op.attend(0, q1, k1, v1).clone()
-        outs[balance] = (dense, sparse)
-        print(f"  balance={balance}: done", flush=True)
-    assert torch.equal(outs[True][0], outs[False][0])
-    assert torch.equal(outs[True][1], outs[False][1])
+        dense[balance] = op.attend(0, q, k, v).clone()
+        print(f"  refresh balance={balance}: done", flush=True)
+    assert ran == [True, False]
+    assert torch.equal(dense[True], dense[False])
+    op.begin_step(1, SPARSE)
+    sparse = op.attend(0, q1, k1, v1)
+    layer, bank = op.layers[0][0], op.banks[0][0]
+    geo, rowmap, scale = op._geometry(q1), op.layout.rowmap(q1.device), K.scale_for(wl.dim)
+    kv = K.kv_pack(k1, v1, rowmap, geo)
+    go, gl, drift = layer.coarse_tail_apply(
+        q1, rowmap, layer.coarse_tail_context(kv, geo),
+        bank.partition.reshape(-1, geo.nb, geo.nb), geo, scale, glref=bank.coarse_lse)
+    for balance in (True, False):
+        merged = K.sparse_merge_attn(q1, kv, rowmap, bank.head_kernel_mask, geo, scale, go, gl,
+                                     bank.value, bank.log_mass, bank.coarse_lse,
+                                     K.drift_center(drift, geo), balance=balance)
+        print(f"  merge balance={balance}, {geo.attn_split} segments a long row: done", flush=True)
+        assert torch.equal(merged, sparse), balance
 
 
 def test_wan_refresh_then_four_drifting_sparse_calls_vs_oracle(cuda):
