@@ -290,6 +290,42 @@ def test_split_long_rows(cuda, n, n_video, d, dtype):
         assert float((long_rows[1] - whole[1]).abs().max()) <= 4e-6
 
 
+@pytest.mark.parametrize("n,n_video,d,dtype", [(700, 600, 128, torch.bfloat16),
+                                               (700, 640, 64, torch.float16)])
+def test_attention_entries_without_a_workspace(cuda, n, n_video, d, dtype):
+    """recap_block_sparse_attn, and recap_sparse_merge_attn with and without a work queue, bit
+    for bit as the launches with a workspace and undivided long rows."""
+    g = torch.Generator().manual_seed(n + d)
+    banks, tb, rows = 2, -(-n // 128), n_video // 128 * 128
+    print(f"case n={n} d={d}", flush=True)
+    q, k, v = (torch.randn(1, banks, n, d, generator=g).to(cuda, dtype) for _ in range(3))
+    kmask = torch.rand(banks, tb, tb, generator=g) > 0.5
+    kmask[:, torch.arange(tb), torch.arange(tb)] = True
+    kmask = kmask.to(cuda)
+    gl, dl, ref = (torch.randn(banks, rows, generator=g).to(cuda) for _ in range(3))
+    go = torch.randn(banks, rows, d, generator=g).to(cuda, dtype)
+    det = torch.randn(banks, rows, d, generator=g).to(cuda, torch.float16)
+    center = torch.randn(banks, generator=g).to(cuda)
+    rowmap = torch.randperm(n, generator=g).to(cuda, torch.int32)
+    geo, scale = K.Geometry(n, n_video, attn_split=1), scale_for(d)
+    kv = K.kv_pack(k, v, rowmap, geo)
+    stream = torch.cuda.current_stream().cuda_stream
+    head, lse = torch.empty(banks, n, d, dtype=dtype, device=cuda), torch.empty(banks, n, device=cuda)
+    common = (q.data_ptr(), K.dtype_code(dtype), 1, banks, d, *q.stride()[:3],
+              kv.k_tiles.data_ptr(), kv.vt_tiles.data_ptr(), rowmap.data_ptr(), kmask.data_ptr(), n)
+    _lib.call("recap_block_sparse_attn", *common, scale, head.data_ptr(), lse.data_ptr(), stream)
+    want, want_lse = K.block_sparse_attn(q, kv, rowmap, kmask, geo, scale)
+    assert torch.equal(head, want) and torch.equal(lse, want_lse)
+    merged = K.sparse_merge_attn(q, kv, rowmap, kmask, geo, scale, go, gl, det, dl, ref, center)
+    for words in (0, int(_lib.load().recap_attn_queue_words())):
+        queue = torch.full((max(1, words),), -1, dtype=torch.int32, device=cuda)
+        out = torch.empty_like(q)
+        _lib.call("recap_sparse_merge_attn", *common, n_video, scale, go.data_ptr(), gl.data_ptr(),
+                  det.data_ptr(), dl.data_ptr(), ref.data_ptr(), center.data_ptr(), -1.0,
+                  out.data_ptr(), *out.stride()[:3], queue.data_ptr() if words else None, stream)
+        assert torch.equal(out, merged), words
+
+
 @pytest.mark.parametrize("d", [64, 128])
 def test_attention_running_max_jumps(cuda, d):
     """Keys of each 64-key sub-tile scaled by factors from 0.1 to 80, so that a row's scores
