@@ -105,7 +105,7 @@ __device__ inline float drift_centre(const float* part, int tiles, int rows) {
 // every access moves 16 bytes.  In merge mode the row's coarse output and refinement are all
 // requested before the first of them is used: with the loads between the stores (which the
 // compiler must keep in order: the output might be one of the inputs) each 8-byte load waited
-// out the memory's latency, 16-18 us a work item of 100-200 us; now 4.
+// out the memory's latency, 16-18 us a work item of 100-200 us; now 5-7.
 template <class T, int D, int MODE>
 __device__ inline void store_rows(const AttnArgs& a, int bank, int b, int h, int r, int nat,
                                   int g, const f32x16 (&oacc)[D / 32], float m, float lt) {
@@ -768,10 +768,10 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
       // Every segment of a long row starts from the running max that the undivided walk has
       // after its first sub-tile: the probabilities, which are rounded to 16 bits relative to
       // it, are then the undivided walk's (but where a segment's scores make it raise the max
-      // again), and only the order of the fp32 sums is another.  From a
-      // max of their own, 9-34% of the long rows' elements came out as the neighbouring value
-      // (12 heads x 7,800 tokens; 12 x 4,856 in fp16), now 0.8-7%; no time to be seen (127.9
-      // us a sparse call at the second, 128.8 before, runs 2.5% apart).
+      // again), and only the order of the fp32 sums is another.  From a max of their own, 9-34%
+      // of the long rows' elements came out as the neighbouring value (12 heads x 7,800 tokens;
+      // 12 x 4,856 in fp16), now 0.8-7%; no time to be seen (127.9 us a sparse call at the
+      // second, 128.8 before, runs 2.5% apart).
       qk(v_lds1, sa);
       if (ragged && __builtin_amdgcn_readfirstlane(list[0]) == a.tb - 1) mask_tail(sa, 0);
       row_max(sa);
@@ -870,11 +870,13 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
 // rows keep about `density` of their blocks.  A long row as one item takes its tb tiles
 // however idle the chip is, so it is cut until a segment is no longer than the other items, or
 // than half of the work there is for each of the 512 workgroups, and not below 16 tiles (a
-// segment's state costs about two tiles to store and combine); and not so far that items which
-// fit one round of the 512 need a second.  Attention kernel, 1 segment -> this rule: 101 -> 73 us
-// at 12 banks of 38 blocks (2 segments; 3: 80, 6: 73), 203 -> 178 us at 12 of 61 (3; 6: 199),
-// 333 -> 275 us at 8 of 125 (4; 6: 276); no change at 12 of 256 (2).  It depends on the layer's
-// sizes only, so that every group of its heads is cut alike.
+// segment's state costs about two tiles to store and combine); and where two segments a row fit
+// one round of the 512, not so far that the items need a second.  (Two segments stay also where
+// the undivided rows alone fit it: 102 us undivided, 71 with two and 70 with the rule's three at
+// 12 banks of 42 blocks, 504, 516 and 528 items.)  Attention kernel, 1 segment -> this rule: 101 ->
+// 73 us at 12 banks of 38 blocks (2 segments; 3: 80, 6: 73), 203 -> 178 us at 12 of 61 (3; 6:
+// 199), 333 -> 275 us at 8 of 125 (4; 6: 276); no change at 12 of 256 (2).  It depends on the
+// layer's sizes only, so that every group of its heads is cut alike.
 int attn_split(int64_t banks, int64_t tb, int64_t ds, double density) {
   if (ds >= tb) return 1;
   const double longs = (double)(tb - ds), other = density * (double)tb + longs + 1.0;

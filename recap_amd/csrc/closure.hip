@@ -469,14 +469,17 @@ hipError_t run_closure(const ClosureArgs& a, int dtype, int dim, int flags, hipS
 // partial (64 KB) are paid for once.  Kernel and sum: 97 us with 1,032 groups of 3 blocks (four
 // rounds and a bit) -> 58 with 240 of 13 at 12 heads x 32,760 tokens; 42 -> 26 at 12 x 7,800 (732
 // of 1 -> 252 of 3); 461 -> 402 at 24 x 119,056 (2,808 of 8 -> 240 of 93).  The four runs let a
-// quarter of the layer's heads, called alone, spread over as many workgroups; longer groups have
-// as many runs as keep each to 24 blocks.  (A run is one chain of fp32 additions.  Relative error of
-// the sums over 929 blocks: 1.5e-7 in groups of 8, 9.4e-8 in groups of 93 with runs of 23, but
-// 1.7e-7 with runs of 47 and 7.3e-7 with runs of 233, four in the longest groups; 1.2e-7
-// with 39 of 24, in the same time.)  More than 256 banks take several rounds whatever the group, and one group a bank would leave the last of them nearly
-// empty (closure and tables 274 us at 300 banks of 61 blocks, d = 64, now 202; 1,111 -> 726 at 300
-// of 256): there the group is the one with the shortest rounds, a workgroup's prologue and
-// partial counted as two blocks (by the figures above).
+// quarter of the layer's heads, called alone, spread over as many workgroups.
+//
+// A run is one chain of fp32 additions, so longer groups have as many as keep each to 24 blocks.
+// Relative error of the sums over 929 blocks: 1.5e-7 in groups of 8 and 9.4e-8 in groups of 93
+// with runs of 23, but 1.7e-7 with runs of 47 and 7.3e-7 with runs of 233 (four in the longest
+// groups); 1.2e-7 at most with this rule, in the same time.
+//
+// More than 256 banks take several rounds whatever the group, and one group a bank would leave
+// the last of them nearly empty (closure and tables 274 us at 300 banks of 61 blocks, d = 64, now
+// 202; 1,111 -> 726 at 300 of 256): there the group is the one with the shortest rounds, a
+// workgroup's prologue and partial counted as two blocks (by the figures above).
 ClosureSpan closure_span(int64_t banks, int64_t nb) {
   int64_t best = 1;
   if (banks > 256) {

@@ -223,8 +223,9 @@ __device__ __forceinline__ bool jacobi_rotation(float app, float aqq, float apq,
   return turn;
 }
 
-// The same sweeps for n = N = 64 or 128 (the head dimensions) with A and V in registers, bit
-// for bit.  Slot k of a round is its pair k; a lane holds one slot's rows (two elements, row p
+// The same sweeps for n = N = 64 or 128 (the head dimensions) with A and V in registers, every
+// element by the operations of the kernel above, which took these orders before (values and vectors
+// compared bit for bit then, on 16 batches: scatters, indefinite, diagonal, rank 3, zero).  Slot k of a round is its pair k; a lane holds one slot's rows (two elements, row p
 // and row q of a column) and a wave eight slots' columns, so a 2 x 2 block (k, l) is in one
 // lane.  From a round to the next the circle ordering moves every column and every row by one
 // slot (q's right, p's left, p of slot 0 staying, q of the last slot turning into its p, p of
