@@ -224,10 +224,11 @@ __device__ __forceinline__ bool jacobi_rotation(float app, float aqq, float apq,
 }
 
 // The same sweeps for n = N = 64 or 128 (the head dimensions) with A and V in registers, every
-// element by the operations of the kernel above, which took these orders before (values and vectors
-// compared bit for bit then, on 16 batches: scatters, indefinite, diagonal, rank 3, zero).  Slot k of a round is its pair k; a lane holds one slot's rows (two elements, row p
-// and row q of a column) and a wave eight slots' columns, so a 2 x 2 block (k, l) is in one
-// lane.  From a round to the next the circle ordering moves every column and every row by one
+// element by the operations of the kernel above, which took these orders before (values and
+// vectors compared bit for bit then, on 16 batches: scatters, indefinite, diagonal, rank 3, zero).
+// Slot k of a round is its pair k; a lane holds one slot's rows (two elements, row p and row q of
+// a column) and a wave eight slots' columns, so a 2 x 2 block (k, l) is in one lane.  From a
+// round to the next the circle ordering moves every column and every row by one
 // slot (q's right, p's left, p of slot 0 staying, q of the last slot turning into its p, p of
 // slot 1 into q of slot 0): rows move by lane shifts, columns by the register renaming of an
 // eightfold unrolled loop, and only the two columns that leave a wave go through LDS, with one
