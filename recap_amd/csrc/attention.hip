@@ -284,8 +284,12 @@ __device__ inline bool merge_segments(const AttnArgs& a, int item, int seg, int 
   return true;
 }
 
+// Starts on a multiple of 16 KB: with cold caches a short launch otherwise depends on where the
+// linker puts the code (the same 40 KB at 0x3600 past such a boundary 83-85 us, at 0x0, 0x1600 and
+// 0x2000 72-76, at 12 heads x 4,856 tokens in fp16; no difference once the code is warm).
 template <class T, int D, int MODE>
-__global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
+__global__ __launch_bounds__(kThreads, 2) __attribute__((aligned(16384)))
+void attention_kernel(AttnArgs a) {
   using G = TileGeom<D>;
   constexpr int NS = D / 16;                  // k-steps over the head dimension
   constexpr int NDT = D / 32;                 // 32-row tiles of O^T
@@ -483,36 +487,18 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
           16 * kThreads * i + 16 * t, off, 0, 0);
   };
 
-  if (nsub > 0) {
-    copy(krs, image(0), k_lds0);
-    if constexpr (D != 64) copy(vrs, image(0), v_lds0);   // (at d = 64 its step copies it)
-  }
-  if (nsub > 1) copy(krs, image(1), k_lds1);
-  // A later segment also gets the K image of the whole row's first sub-tile (see below).
-  if (kSplits && seg > 0 && nsub > 0)
-    copy(krs, __builtin_amdgcn_readfirstlane(list[0] * G::kTileBytes), v_lds1);
-  tile_barrier();
-
-  float m[kGroups], mraw[kGroups], lsum[kGroups];
   const float inv_scale_log2 = 1.0f / a.scale_log2;
-  f32x16 oacc[kGroups][NDT];
-#pragma unroll
-  for (int q = 0; q < kGroups; ++q) {
-    m[q] = -INFINITY;
-    mraw[q] = -INFINITY;
-    lsum[q] = 0.0f;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) oacc[q][dt] = f32x16{};
-  }
   const bool ragged = (a.n_tokens % kBlock) != 0;
 
-  // S^T (64 keys x 32 queries of each group) of the sub-tile whose K image is in `kl`.
-  auto qk = [&](const char* kl, f32x16 (&s)[kGroups][2]) {
+  // S^T (64 keys x 32 queries of each group) of the sub-tile whose K image is in `kl`, by the lane's
+  // row and half (l32 and g; captured, they had the compiler compute eight of the main walk's LDS
+  // addresses anew in every pair of steps, 1% at 24 heads x 119,056 tokens).
+  auto qk = [&](const char* kl, f32x16 (&s)[kGroups][2], int lr, int lg) {
 #pragma unroll
     for (int st = 0; st < NS; ++st)
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt) {
-        const u32x4 ka = lds_load16(kl, G::k_off(32 * kt + l32, 2 * st + g));
+        const u32x4 ka = lds_load16(kl, G::k_off(32 * kt + lr, 2 * st + lg));
 #pragma unroll
         for (int q = 0; q < kGroups; ++q)
           s[q][kt] = T::mfma32(ka, qreg[q][st], st == 0 ? f32x16{} : s[q][kt]);
@@ -527,9 +513,32 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int rr = 0; rr < 16; ++rr)
+        for (int rr = 0; rr < 16; ++rr) {
+          // At d = 64 also one at a time: 32 masks at once took the scalar registers that the walk
+          // keeps its copies' LDS addresses in (0.8% at 48 heads x 45,106 tokens; at d = 128 the
+          // walk is scheduled better with them at once, 0.5% at 24 x 119,056).
+          if constexpr (D == 64) asm volatile("" : "+v"(limit));
           if (32 * kt + mfma_row(rr, 0) >= limit) s[q][kt][rr] = -INFINITY;
+        }
   };
+  auto lane_max = [](f32x16 (&s)[2]) {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr) mx = __builtin_elementwise_maximum(mx, s[kt][rr]);
+    return mx;
+  };
+  float m[kGroups], mraw[kGroups], lsum[kGroups];
+  f32x16 oacc[kGroups][NDT];
+#pragma unroll
+  for (int q = 0; q < kGroups; ++q) {
+    m[q] = -INFINITY;
+    mraw[q] = -INFINITY;
+    lsum[q] = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) oacc[q][dt] = f32x16{};
+  }
   // Lazy running-max update of group q from a per-lane candidate raw score: moves only when
   // the row max grows by more than kRescaleSlack, rescaling O and l.  The test is on raw
   // scores against mraw = (m + slack) / (scale log2 e), kept with m (scale > 0).
@@ -544,17 +553,6 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
       for (int dt = 0; dt < NDT; ++dt) oacc[q][dt] *= alpha;
       m[q] = mnew;
       mraw[q] = (mnew + kRescaleSlack) * inv_scale_log2;
-    }
-  };
-  auto row_max = [&](f32x16 (&s)[kGroups][2]) {
-#pragma unroll
-    for (int q = 0; q < kGroups; ++q) {
-      float mx = -INFINITY;
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int rr = 0; rr < 16; ++rr) mx = __builtin_elementwise_maximum(mx, s[q][kt][rr]);
-      update_max(q, mx);
     }
   };
 
@@ -763,23 +761,33 @@ __global__ __launch_bounds__(kThreads, 2) void attention_kernel(AttnArgs a) {
   };
 
   f32x16 sa[kGroups][2], sb[kGroups][2];
-  if (nsub > 0) {
-    if (kSplits && seg > 0) {
-      // Every segment of a long row starts from the running max that the undivided walk has
-      // after its first sub-tile: the probabilities, which are rounded to 16 bits relative to
-      // it, are then the undivided walk's (but where a segment's scores make it raise the max
-      // again), and only the order of the fp32 sums is another.  From a max of their own, 9-34%
-      // of the long rows' elements came out as the neighbouring value (12 heads x 7,800 tokens;
-      // 12 x 4,856 in fp16), now 0.8-7%; no time to be seen (127.9 us a sparse call at the
-      // second, 128.8 before, runs 2.5% apart).
-      qk(v_lds1, sa);
-      if (ragged && __builtin_amdgcn_readfirstlane(list[0]) == a.tb - 1) mask_tail(sa, 0);
-      row_max(sa);
+  // The walk's first scores and running max.  Every segment of a long row starts from the max that
+  // the undivided walk has after its first sub-tile: a later segment takes the scores of that one
+  // (pass 0) before those of its own (pass 1).  The probabilities, which are rounded to 16 bits
+  // relative to the max, are then the undivided walk's (but where a segment's scores make it raise
+  // the max again), and only the order of the fp32 sums is another.  From a max of their own, 9-34%
+  // of the long rows' elements came out as the neighbouring value (12 heads x 7,800 tokens; 12 x
+  // 4,856 in fp16), now 0.8-7%, in the same time.
+#pragma unroll 1
+  for (int pass = kSplits && first > 0 ? 0 : 1; pass < 2 && nsub > 0; ++pass) {
+    const int j = MODE == kModeDense ? 0 : __builtin_amdgcn_readfirstlane(list[pass == 0 ? 0 : first]);
+    copy(krs, j * G::kTileBytes, k_lds0);
+    if (pass == 1) {
+      if constexpr (D != 64) copy(vrs, image(0), v_lds0);   // (at d = 64 its step copies it)
+      if (nsub > 1) copy(krs, image(1), k_lds1);
     }
-    qk(k_lds0, sa);
-    if (ragged_at(0)) mask_tail(sa, 0);
-    row_max(sa);
-    tile_barrier();  // the first steps overwrite K slot 0 and V slot 1 (read just now)
+    tile_barrier();
+    qk(k_lds0, sa, l32, g);
+    if (ragged && j == a.tb - 1) mask_tail(sa, 0);
+#pragma unroll
+    for (int q = 0; q < kGroups; ++q) {
+      const float pm = pair_max(lane_max(sa[q]));
+      if (pm > mraw[q] && (D != 64 || m[q] == -INFINITY)) {
+        m[q] = pm * a.scale_log2;
+        if constexpr (D != 64) mraw[q] = (m[q] + kRescaleSlack) * inv_scale_log2;
+      }
+    }
+    tile_barrier();  // K slot 0 is copied over next
   }
   using F = std::false_type;
   using Tr = std::true_type;

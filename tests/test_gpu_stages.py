@@ -366,6 +366,34 @@ def test_attention_running_max_jumps(cuda, d):
         assert bool((err <= bound).all()), float((err - bound).max())
 
 
+@pytest.mark.parametrize("d", [64, 128])
+def test_split_long_rows_running_max_jumps(cuda, d):
+    """Segments of long rows whose scores rise by tens of log2 units within and between the
+    segments, from the running max of the row's first sub-tile (which keeps the smallest keys):
+    output and LSE against the oracle for one to eight segments, bounds as above."""
+    n, banks = 1000, 2
+    print(f"case n={n} d={d}", flush=True)
+    g = torch.Generator().manual_seed(29 + d)
+    tb = -(-n // 128)
+    q, k, v = (torch.randn(1, banks, n, d, generator=g) for _ in range(3))
+    factors = torch.tensor([0.1, 1.0, 8.0, 0.25, 24.0, 2.0, 40.0, 0.5, 12.0, 3.0, 60.0, 1.0, 80.0,
+                            16.0, 0.1, 5.0])
+    k = k * factors[torch.arange(n) // 64].view(1, 1, n, 1)
+    q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    kmask = torch.ones(banks, tb, tb, dtype=torch.bool)
+    kmask[0, :, -1] = False    # opens with the small keys; the other head with the ragged block
+    rowmap = torch.arange(n, dtype=torch.int32, device=cuda)
+    kv = K.kv_pack(k.to(cuda), v.to(cuda), rowmap, K.Geometry(n, n))
+    scale = scale_for(d)
+    ref, ref_lse = O.block_sparse_attention(*(x[0].float() for x in (q, k, v)), kmask, scale)
+    for split in (1, 2, 3, 8):
+        geo = K.Geometry(n, 128, attn_split=split)   # every row but the first block's is long
+        head, lse = K.block_sparse_attn(q.to(cuda), kv, rowmap, kmask.to(cuda), geo, scale)
+        assert_parity(head.cpu().float(), ref, f"split {split}")
+        err = (lse.cpu().double() - ref_lse.double()).abs()
+        assert bool((err <= 2e-3 + 1e-5 * ref_lse.double().abs()).all()), float(err.max())
+
+
 def test_dense_attention_matches_torch_sdpa(cuda):
     wl = SMALL["text-last-d128"]
     q, k, v = (x.to(cuda) for x in make_qkv(wl, seed=1))
