@@ -703,7 +703,7 @@ def test_block_scores_tiles(cuda, banks, nb, d):
                                         ("text-first-ragged", torch.float16),
                                         ("text-last-d128", torch.bfloat16),
                                         ("video-ragged-d128", torch.float16)])
-@pytest.mark.parametrize("span", [(1, 1), (3, 2), (5, 4), (64, 4), (64, 64)])
+@pytest.mark.parametrize("span", [(1, 1), (3, 2), (5, 4), (5, 64), (64, 4), (64, 64)])
 def test_closure_tables_spans(cuda, name, dtype, span):
     """C_vk over groups of one to all blocks in one to 64 runs (empty ones among them): the
     variances and tables bit for bit those of the separate calls, C_vk within the rounding of
